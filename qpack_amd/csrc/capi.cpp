@@ -262,14 +262,14 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
     need(q, "q"); need(scale, "scale"); need(X, "X"); need(Y, "Y");
     if (rows <= 0 || B <= 0 || cols <= 0 || cols % 128) throw std::invalid_argument("matmul: rows, B > 0 and cols a positive multiple of 128 required");
     if (kind != QPH_Q8 && kind != QPH_Q4) throw std::invalid_argument("matmul: kind must be QPH_Q8 or QPH_Q4");
-    const int nb = cols / 128, G = cols / 32, ldg = (G + 3) / 4 * 4;
+    const int nb = cols / 128, ldb = (nb + 7) / 8 * 8, G = cols / 32, ldg = (G + 3) / 4 * 4;
     const size_t qb = kind == QPH_Q8 ? (size_t)rows * cols : (size_t)rows * cols / 2;
     const size_t sb = kind == QPH_Q8 ? 4ull * rows : 2ull * rows * G;
     std::vector<void *> bufs;
     auto alloc = [&](size_t n) { void *p = nullptr; hck(hipMalloc(&p, n), "hipMalloc"); bufs.push_back(p); return p; };
     try {
       void *dq = alloc(qb), *ds = alloc(sb);
-      float *dx = (float *)alloc(4ull * B * cols), *dy = (float *)alloc(4ull * B * rows), *dxb = (float *)alloc(4ull * B * nb);
+      float *dx = (float *)alloc(4ull * B * cols), *dy = (float *)alloc(4ull * B * rows), *dxb = (float *)alloc(4ull * B * ldb);
       const int ldbt = (B + 63) / 64 * 64;
       float *dxbt = (float *)alloc(4ull * ldbt * nb);
       int8_t *dxh = (int8_t *)alloc((size_t)B * cols), *dxl = (int8_t *)alloc((size_t)B * cols);
@@ -277,12 +277,17 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
       hck(hipMemcpy(dq, q, qb, hipMemcpyHostToDevice), "upload q");
       hck(hipMemcpy(ds, scale, sb, hipMemcpyHostToDevice), "upload scale");
       hck(hipMemcpy(dx, X, 4ull * B * cols, hipMemcpyHostToDevice), "upload X");
-      qph::PfQuantArgs qa{}; qa.x = dx; qa.ldx = cols; qa.cols = cols; qa.xh = dxh; qa.xl = dxl; qa.ldq = cols; qa.xb = dxb; qa.ldb = nb;
-      qa.xg = dxg; qa.ldg = ldg; qa.xbt = dxbt; qa.ldbt = ldbt;
-      hck(qph::launch_pf_quant(qph::PRO_QUANT, qa, B, nullptr), "launch quant");
       qph::GemmArgs ga{}; ga.kind = kind == QPH_Q8 ? qph::MK_Q8 : qph::MK_Q4; ga.w = (const int8_t *)dq; ga.scale = (const float *)ds;
-      ga.rows = rows; ga.cols = cols; ga.xh = dxh; ga.xl = dxl; ga.xb = dxb; ga.ntok = B; ga.ldq = cols; ga.ldb = nb;
+      ga.rows = rows; ga.cols = cols; ga.xh = dxh; ga.xl = dxl; ga.xb = dxb; ga.ntok = B; ga.ldq = cols; ga.ldb = ldb;
       ga.xg = dxg; ga.ldg = ldg; ga.y = dy; ga.ldy = rows; ga.xbt = dxbt; ga.ldbt = ldbt;
+      qph::PfQuantArgs qa{}; qa.x = dx; qa.ldx = cols; qa.cols = cols; qa.xh = dxh; qa.xl = dxl; qa.ldq = cols; qa.xb = dxb; qa.ldb = ldb;
+      qa.xg = dxg; qa.ldg = ldg; qa.xbt = dxbt; qa.ldbt = ldbt;
+      if (qph::gemm_wants_tiles(ga)) {   // the few-token kernel: the planes in 16-token tiles
+        const size_t tb = (size_t)(B + 15) / 16 * 16 * cols;
+        qa.th = (int8_t *)alloc(tb); qa.tl = (int8_t *)alloc(tb); qa.xh = qa.xl = nullptr;
+        ga.th = qa.th; ga.tl = qa.tl;
+      }
+      hck(qph::launch_pf_quant(qph::PRO_QUANT, qa, B, nullptr), "launch quant");
       if (kind == QPH_Q8) {
         int *dws = (int *)alloc(4ull * qph::ws_pitch(rows) * nb);
         hck(qph::launch_rowsum_q8((const int8_t *)dq, rows, cols, dws, nullptr), "launch rowsum");

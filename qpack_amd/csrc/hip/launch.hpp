@@ -178,6 +178,10 @@ struct PfQuantArgs {
   float *xb; int ldb;
   float *xbt; int ldbt;   // optional: the block scales block-major [cols / 128][ldbt]
   int *xg; int ldg;   // optional: sum of q per 32-column group [B][ldg] (the q4 product needs it)
+  // optional: the planes again in the order the few-token products read them (k_skinny_q8): per 16-token tile (16 ldq
+  // bytes apart) the 16-column piece p of each 128-column block (2048 bytes) of token t at byte
+  // 1024 (p % 2) + 256 (p / 2) + 16 (t % 16)
+  int8_t *th, *tl;
 };
 hipError_t launch_pf_quant(int pro, const PfQuantArgs &a, int B, hipStream_t st);
 // Y[t][r] = the row's dot product with token t's quantised activation (+ bias[r]), or Y[t][r] += that when resid.
@@ -197,6 +201,7 @@ struct GemmArgs {
   const int *q4ns; const float *q4sc;
   const int *xg; int ldg;
   const int8_t *xh, *xl; const float *xb; int ntok, ldq, ldb;
+  const int8_t *th, *tl;   // optional (q8): the planes in 16-token tiles (PfQuantArgs::th), whole tiles allocated
   const float *xbt; int ldbt;   // q8: the block scales again, block-major [cols / 128][ldbt] (ldbt % 4 == 0, >= ntok)
   float *y; int ldy;
   const float *bias;
@@ -225,9 +230,17 @@ __host__ __device__ inline int ws_pitch(int rows) { return (rows + 63) & ~63; }
 hipError_t launch_rowsum_q8(const int8_t *w, int rows, int cols, int *out, hipStream_t st);
 // q4 rows: per (block, group, row) the sum of the nibbles and the f32 scale, group-major within each 128-column block
 hipError_t launch_q4_prep(const uint8_t *w, const uint16_t *sc, int rows, int cols, int *out_ns, float *out_sc, hipStream_t st);
+// launch_gemm runs a q8 launch with th set on the few-token kernel, others on the tiled ones (which read xh / xl);
+// gemm_wants_tiles: whether th is the faster choice for this product (the pointers need not be set yet)
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t st);
+bool gemm_wants_tiles(const GemmArgs &a);
 // whether launch_gemm runs this q8 launch on the 32 x 32 kernel (the one that can quantise a SwiGLU pair's output)
 bool gemm_uses_32x32(const GemmArgs &a);
+// q8 products of few tokens or few rows (skinny.hip): K split over the waves of a workgroup of 16 rt rows (16 of each
+// matrix for a gate / up pair, rt = 2) x 16 ntt tokens; reads the planes from th / tl; ldb a multiple of 8
+hipError_t launch_skinny(const GemmArgs &a, int rt, int ntt, int cus, hipStream_t st);
+// its best tile for this product and the microseconds that is expected to take
+double skinny_cost(const GemmArgs &a, int cus, int *rt, int *ntt);
 // token t of the batch at position p0 + t: RoPE on q [t][ldq] (in place) and k, fp16 k / v rows into the caches
 struct PfRopeArgs {
   float *q; int ldq;
@@ -246,6 +259,7 @@ struct PfAttnArgs {
   int ntok, p0, nh, nkv, hd;
   // optional: q not yet rotated - the kernel applies RoPE (k_pf_rope's arithmetic) as it loads q
   const float *cos_t, *sin_t;
+  int tiled;   // oh / ol in 16-token tiles (PfQuantArgs::th), not rows
   // optional (hd 128, one head = one 128-column block): the output quantised for the wo product instead of att -
   // planes oh / ol [ntok][ldo], block scales ob [ntok][ldb] and obt [nh][ldbt] (the quantiser's arithmetic)
   int8_t *oh, *ol; float *ob, *obt; int ldo, ldb, ldbt;

@@ -206,10 +206,13 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
     pf_g_ = (float *)dalloc(4 * B * ff);
     pf_xh_ = (int8_t *)dalloc(B * pf_ldq_); pf_xl_ = (int8_t *)dalloc(B * pf_ldq_);
     pf_xh2_ = (int8_t *)dalloc(B * pf_ldq_); pf_xl2_ = (int8_t *)dalloc(B * pf_ldq_);   // the SwiGLU output, quantised
-    pf_xb_ = (float *)dalloc(4 * B * (pf_ldq_ / 128 + 1));
+    const size_t B16 = (B + 15) / 16 * 16;
+    pf_th_ = (int8_t *)dalloc(B16 * pf_ldq_); pf_tl_ = (int8_t *)dalloc(B16 * pf_ldq_);
+    pf_ldb_ = ((int)wide / 128 + 7) / 8 * 8;   // whole 8-block rounds, 16-byte aligned
+    pf_xb_ = (float *)dalloc(4 * B * pf_ldb_);
     pf_ldbt_ = (int)(B + 63) / 64 * 64;
     pf_xbt_ = (float *)dalloc(4ull * pf_ldbt_ * (pf_ldq_ / 128 + 1));
-    pf_xb2_ = (float *)dalloc(4 * B * (pf_ldq_ / 128 + 1));
+    pf_xb2_ = (float *)dalloc(4 * B * pf_ldb_);
     pf_xbt2_ = (float *)dalloc(4ull * pf_ldbt_ * (pf_ldq_ / 128 + 1));
     pf_ldg_ = (pf_ldq_ / 32 + 3) / 4 * 4;
     pf_xg_ = (int *)dalloc(4 * B * pf_ldg_);
@@ -530,39 +533,55 @@ void HipLlama::prefill_batched(const int *toks, int n) {
   // QPH_PF_UNFUSED=bits (test hook): 1 q's RoPE, 2 the attention output's quantisation, 4 the SwiGLU output's
   // quantisation as launches of their own, for bit-for-bit comparisons with the fused kernels
   const int unfused = getenv("QPH_PF_UNFUSED") ? atoi(getenv("QPH_PF_UNFUSED")) : 0;
-  const int d = cfg_.hidden, ff = cfg_.ffn, nb_ld = pf_ldq_ / 128 + 1;
+  const int d = cfg_.hidden, ff = cfg_.ffn, nb_ld = pf_ldb_;
   const float eps = cfg_.rms_eps;
-  auto quant = [&](int pro, const float *x, int ldx, const float *w, int cols, int B) {
+  // the products of one activation, first planned (which planes does each read), then quantised for, then launched
+  struct Planes { bool rows, tiles; };
+  auto plan = [&](GemmArgs *g, int ng) {
+    Planes p{false, false};
+    for (int i = 0; i < ng; i++) {
+      if (gemm_wants_tiles(g[i])) { g[i].th = pf_th_; g[i].tl = pf_tl_; p.tiles = true; }
+      else p.rows = true;
+    }
+    return p;
+  };
+  auto quant = [&](int pro, const float *x, int ldx, const float *w, int cols, int B, Planes p) {
     PfQuantArgs a{}; a.x = x; a.ldx = ldx; a.norm_w = w; a.eps = eps; a.cols = cols;
-    a.xh = pf_xh_; a.xl = pf_xl_; a.ldq = pf_ldq_; a.xb = pf_xb_; a.ldb = nb_ld; a.xg = pf_xg_; a.ldg = pf_ldg_;
+    if (p.rows) { a.xh = pf_xh_; a.xl = pf_xl_; }
+    if (p.tiles) { a.th = pf_th_; a.tl = pf_tl_; }
+    a.ldq = pf_ldq_; a.xb = pf_xb_; a.ldb = nb_ld; a.xg = pf_xg_; a.ldg = pf_ldg_;
     a.xbt = pf_xbt_; a.ldbt = pf_ldbt_;
     QPH_CK(launch_pf_quant(pro, a, B, st_));
   };
-  auto gemm = [&](const DMat &m, float *y, int ldy, const float *bias, bool resid, int B, const float *gate = nullptr) {
-    GemmArgs a{}; a.kind = m.kind; a.w = (const int8_t *)m.q; a.scale = (const float *)m.s; a.rows = m.rows; a.cols = m.cols;
-    a.wsum = m.rs; a.xbt = pf_xbt_; a.ldbt = pf_ldbt_; a.q4ns = m.q4ns; a.q4sc = m.q4sc; a.xg = pf_xg_; a.ldg = pf_ldg_;
+  auto operands = [&](int kind, int cols, int B) {
+    GemmArgs a{}; a.kind = kind; a.cols = cols; a.xbt = pf_xbt_; a.ldbt = pf_ldbt_; a.xg = pf_xg_; a.ldg = pf_ldg_;
     a.xh = pf_xh_; a.xl = pf_xl_; a.xb = pf_xb_; a.ntok = B; a.ldq = pf_ldq_; a.ldb = nb_ld;
-    a.y = y; a.ldy = ldy; a.bias = bias; a.resid = resid ? 1 : 0; a.gate = gate;
-    QPH_CK(launch_gemm(a, st_));
+    return a;
+  };
+  auto product = [&](const DMat &m, float *y, int ldy, const float *bias, bool resid, int B, const float *gate = nullptr) {
+    GemmArgs a = operands(m.kind, m.cols, B); a.w = (const int8_t *)m.q; a.scale = (const float *)m.s; a.rows = m.rows;
+    a.wsum = m.rs; a.q4ns = m.q4ns; a.q4sc = m.q4sc; a.y = y; a.ldy = ldy; a.bias = bias; a.resid = resid ? 1 : 0; a.gate = gate;
+    return a;
   };
   // q / k / v: runs of consecutive matrices of one kind share a launch (q8 files: one launch; q4m: q + k, then v)
-  auto gemm_qkv = [&](const Layer &ly, int B) {
+  auto qkv = [&](const Layer &ly, int B, GemmArgs *g) {
     const DMat *m[3] = {&ly.wq, &ly.wk, &ly.wv};
     float *y[3] = {pf_q_, pf_k_, pf_v_};
     const int ld[3] = {qd_, kvd_, kvd_};
     const float *bias[3] = {ly.bq, ly.bk, ly.bv};
+    int ng = 0;
     for (int i = 0; i < 3;) {
       int j = i + 1;
       while (j < 3 && m[j]->kind == m[i]->kind && m[j]->cols == m[i]->cols) j++;
-      if (j - i == 1 || (m[i]->kind != MK_Q8 && m[i]->kind != MK_Q4)) { gemm(*m[i], y[i], ld[i], bias[i], false, B); i++; continue; }
-      GemmArgs a{}; a.kind = m[i]->kind; a.cols = m[i]->cols; a.xbt = pf_xbt_; a.ldbt = pf_ldbt_; a.xg = pf_xg_; a.ldg = pf_ldg_;
-      a.xh = pf_xh_; a.xl = pf_xl_; a.xb = pf_xb_; a.ntok = B; a.ldq = pf_ldq_; a.ldb = nb_ld;
+      if (j - i == 1 || (m[i]->kind != MK_Q8 && m[i]->kind != MK_Q4)) { g[ng++] = product(*m[i], y[i], ld[i], bias[i], false, B); i++; continue; }
+      GemmArgs a = operands(m[i]->kind, m[i]->cols, B);
       a.nseg = j - i;
       for (int s = i; s < j; s++)
         a.seg[s - i] = GemmSeg{(const int8_t *)m[s]->q, (const float *)m[s]->s, m[s]->rs, m[s]->q4ns, m[s]->q4sc, bias[s], y[s], m[s]->rows, ld[s]};
-      QPH_CK(launch_gemm(a, st_));
+      g[ng++] = a;
       i = j;
     }
+    return ng;
   };
   int B = 0;
   for (int s0 = 0; s0 < n; s0 += B) {
@@ -573,8 +592,10 @@ void HipLlama::prefill_batched(const int *toks, int n) {
     for (int l = 0; l < cfg_.layers; l++) {
       const Layer &ly = layers_[l];
       uint16_t *kc = kc_ + (size_t)l * ctx_ * kvd_, *vc = vc_ + (size_t)l * ctx_ * kvd_;
-      quant(PRO_NORM, pf_x_, d, ly.an, d, B);
-      gemm_qkv(ly, B);
+      GemmArgs g[3];
+      int ng = qkv(ly, B, g);
+      quant(PRO_NORM, pf_x_, d, ly.an, d, B, plan(g, ng));
+      for (int i = 0; i < ng; i++) QPH_CK(launch_gemm(g[i], st_));
       // q's RoPE happens in the attention kernel; at head dim 128 (one head = one quantisation block) that kernel also
       // quantises its output for a q8 wo
       PfRopeArgs r{}; r.q = pf_q_; r.ldq = qd_; r.k = pf_k_; r.v = pf_v_; r.ldk = kvd_; r.cos_t = cos_; r.sin_t = sin_;
@@ -584,35 +605,39 @@ void HipLlama::prefill_batched(const int *toks, int n) {
       t.ntok = B; t.p0 = p0; t.nh = cfg_.heads; t.nkv = cfg_.kv_heads; t.hd = cfg_.head_dim;
       if (!(unfused & 1)) { t.cos_t = cos_; t.sin_t = sin_; }
       const bool att_q = !(unfused & 2) && cfg_.head_dim == 128 && ly.wo.kind == MK_Q8;
+      g[0] = product(ly.wo, pf_x_, d, nullptr, true, B);
+      Planes pl = plan(g, 1);
       if (att_q) {
-        t.oh = pf_xh_; t.ol = pf_xl_; t.ob = pf_xb_; t.obt = pf_xbt_; t.ldo = pf_ldq_; t.ldb = nb_ld; t.ldbt = pf_ldbt_;
+        t.tiled = pl.tiles;
+        t.oh = pl.tiles ? pf_th_ : pf_xh_; t.ol = pl.tiles ? pf_tl_ : pf_xl_; t.ob = pf_xb_; t.obt = pf_xbt_; t.ldo = pf_ldq_; t.ldb = nb_ld; t.ldbt = pf_ldbt_;
       }
       QPH_CK(launch_pf_attn(t, st_));
-      if (!att_q) quant(PRO_QUANT, pf_att_, qd_, nullptr, qd_, B);
-      gemm(ly.wo, pf_x_, d, nullptr, true, B);
-      quant(PRO_NORM, pf_x_, d, ly.fn, d, B);
+      if (!att_q) quant(PRO_QUANT, pf_att_, qd_, nullptr, qd_, B, pl);
+      QPH_CK(launch_gemm(g[0], st_));
       bool fused = false;   // h = silu(gate) * up quantised by the product's store, straight into the second planes
       if (ly.wg.kind == MK_Q8 && ly.wu.kind == MK_Q8) {   // gate and up in one launch, only h = silu(gate) * up stored
-        GemmArgs a{}; a.kind = MK_Q8; a.w = (const int8_t *)ly.wg.q; a.scale = (const float *)ly.wg.s; a.wsum = ly.wg.rs;
+        GemmArgs &a = g[0];
+        a = product(ly.wg, pf_g_, ff, nullptr, false, B);
         a.w2 = (const int8_t *)ly.wu.q; a.scale2 = (const float *)ly.wu.s; a.wsum2 = ly.wu.rs;
-        a.rows = ff; a.cols = d; a.xbt = pf_xbt_; a.ldbt = pf_ldbt_; a.xh = pf_xh_; a.xl = pf_xl_; a.xb = pf_xb_; a.ntok = B;
-        a.ldq = pf_ldq_; a.ldb = nb_ld; a.y = pf_g_; a.ldy = ff;
-        fused = !(unfused & 4) && ly.wd.kind == MK_Q8 && ff % 128 == 0 && gemm_uses_32x32(a);
+        pl = plan(&a, 1);
+        quant(PRO_NORM, pf_x_, d, ly.fn, d, B, pl);
+        fused = !(unfused & 4) && ly.wd.kind == MK_Q8 && ff % 128 == 0 && !pl.tiles && gemm_uses_32x32(a) &&
+                !gemm_wants_tiles(product(ly.wd, pf_x_, d, nullptr, true, B));
         if (fused) { a.oh = pf_xh2_; a.ol = pf_xl2_; a.ob = pf_xb2_; a.obt = pf_xbt2_; }
         QPH_CK(launch_gemm(a, st_));
       } else {
-        gemm(ly.wg, pf_g_, ff, nullptr, false, B);
-        gemm(ly.wu, pf_g_, ff, nullptr, false, B, pf_g_);   // h = silu(gate) * up, in place over the gate product
+        g[0] = product(ly.wg, pf_g_, ff, nullptr, false, B);
+        g[1] = product(ly.wu, pf_g_, ff, nullptr, false, B, pf_g_);   // h = silu(gate) * up, in place over the gate product
+        quant(PRO_NORM, pf_x_, d, ly.fn, d, B, plan(g, 2));
+        for (int i = 0; i < 2; i++) QPH_CK(launch_gemm(g[i], st_));
       }
+      g[0] = product(ly.wd, pf_x_, d, nullptr, true, B);
       if (fused) {
-        GemmArgs a{}; a.kind = MK_Q8; a.w = (const int8_t *)ly.wd.q; a.scale = (const float *)ly.wd.s; a.rows = ly.wd.rows;
-        a.cols = ly.wd.cols; a.wsum = ly.wd.rs; a.xbt = pf_xbt2_; a.ldbt = pf_ldbt_; a.xh = pf_xh2_; a.xl = pf_xl2_;
-        a.xb = pf_xb2_; a.ntok = B; a.ldq = pf_ldq_; a.ldb = nb_ld; a.y = pf_x_; a.ldy = d; a.resid = 1;
-        QPH_CK(launch_gemm(a, st_));
+        g[0].xh = pf_xh2_; g[0].xl = pf_xl2_; g[0].xb = pf_xb2_; g[0].xbt = pf_xbt2_;
       } else {
-        quant(PRO_QUANT, pf_g_, ff, nullptr, ff, B);
-        gemm(ly.wd, pf_x_, d, nullptr, true, B);
+        quant(PRO_QUANT, pf_g_, ff, nullptr, ff, B, plan(g, 1));
       }
+      QPH_CK(launch_gemm(g[0], st_));
     }
     pos_ += B;
   }
@@ -720,7 +745,7 @@ void HipLlama::ex_norm(const float *x, const float *w, float *out, int rows, int
 // planes first unless `quantised` says they already hold it
 void HipLlama::ex_product(const DMat &m, const float *x, int ldx, int ntok, int mm_below, float *y, int ldy,
                           const float *bias, bool resid, bool quantised) {
-  const int nb_ld = pf_ldq_ / 128 + 1;
+  const int nb_ld = pf_ldb_;
   if (!quantised) {
     PfQuantArgs q{}; q.x = x; q.ldx = ldx; q.cols = m.cols; q.xh = pf_xh_; q.xl = pf_xl_; q.ldq = pf_ldq_;
     q.xb = pf_xb_; q.ldb = nb_ld;

@@ -147,6 +147,8 @@ class HipLlama {
   float *pf_xb_ = nullptr, *pf_xbt_ = nullptr;   // block scales token-major [B][nb], block-major [nb][pf_ldbt_]
   int pf_ldbt_ = 0;
   int8_t *pf_xh_ = nullptr, *pf_xl_ = nullptr;
+  int8_t *pf_th_ = nullptr, *pf_tl_ = nullptr;   // the planes in 16-token tiles (PfQuantArgs::th)
+  int pf_ldb_ = 0;                               // row pitch of the block scales
   int8_t *pf_xh2_ = nullptr, *pf_xl2_ = nullptr;   // second planes: the SwiGLU output quantised by the gate / up store
   float *pf_xb2_ = nullptr, *pf_xbt2_ = nullptr;
   int *pf_tok_ = nullptr, *pf_xg_ = nullptr;

@@ -45,11 +45,16 @@ __global__ __launch_bounds__(1024) void k_pf_quant(PfQuantArgs a) {
   ActRegs ar;
   act_load<PRO>(a.x + (size_t)t * a.ldx, a.norm_w, cols, ar);
   act_build<PRO>(ar, a.eps, cols, av);
-  int8_t *xh = a.xh + (size_t)t * a.ldq, *xl = a.xl + (size_t)t * a.ldq;
+  const size_t trow = (size_t)t * a.ldq, ttile = (size_t)(t & ~15) * a.ldq + 16 * (t & 15);
   for (int c = threadIdx.x * 16; c < cols; c += blockDim.x * 16) {
-    const uint4 h = *(const uint4 *)(av.xh + c), l = *(const uint4 *)(av.xl + c);
-    *(uint4 *)(xh + c) = h;
-    *(uint4 *)(xl + c) = make_uint4(l.x ^ 0x80808080u, l.y ^ 0x80808080u, l.z ^ 0x80808080u, l.w ^ 0x80808080u);
+    const uint4 h = *(const uint4 *)(av.xh + c);
+    uint4 l = *(const uint4 *)(av.xl + c);
+    l = make_uint4(l.x ^ 0x80808080u, l.y ^ 0x80808080u, l.z ^ 0x80808080u, l.w ^ 0x80808080u);
+    if (a.xh) { *(uint4 *)(a.xh + trow + c) = h; *(uint4 *)(a.xl + trow + c) = l; }
+    if (a.th) {
+      const int p = c / 16, o = ((p & ~7) + 4 * (p & 1) + ((p >> 1) & 3)) * 256;
+      *(uint4 *)(a.th + ttile + o) = h; *(uint4 *)(a.tl + ttile + o) = l;
+    }
   }
   for (int b = threadIdx.x; b < nb; b += blockDim.x) a.xb[(size_t)t * a.ldb + b] = av.bs[b];
   if (a.xbt)
@@ -59,7 +64,7 @@ __global__ __launch_bounds__(1024) void k_pf_quant(PfQuantArgs a) {
 }
 hipError_t launch_pf_quant(int pro, const PfQuantArgs &a, int B, hipStream_t st) {
   if (B <= 0) return hipSuccess;
-  if (a.cols % kQB || a.cols > 32768 || a.ldq % 16) return hipErrorInvalidValue;
+  if (a.cols % kQB || a.cols > 32768 || a.ldq % 16 || (!a.xh && !a.th)) return hipErrorInvalidValue;
   const size_t lds = mv_lds_bytes(a.cols, 16, 0);
   // the fewest threads whose two act_load passes cover the row (8 per 128-column block and pass): small workgroups,
   // so several tokens' load -> reduce -> store chains overlap on a CU
@@ -889,11 +894,11 @@ __global__ __launch_bounds__(512) void k_gemm_q4(GemmArgs a) {
 // q8: which product kernel.  A 32 x 32 workgroup does twice a 16 x 16 one's work in ~1.45 x its time (C4 shapes on
 // MI355X: 2 x 14336 x 4096 578 vs 707 us, 4096 x 4096 173 vs 215, 6144 x 4096 152 vs 160), so it wins unless its fewer,
 // larger workgroups leave CUs idle: ceil(n2 / CUs) x 1.45 against ceil(2 n2 / CUs) rounds (n2 = its workgroup count).
-// QPH_GEMM=1 / 2 forces the 32 x 32 / 16 x 16 kernel.
+// QPH_GEMM=1 / 2 / 3 forces the 32 x 32 / 16 x 16 / few-token kernel.
 static int gemm_forced() {   // QPH_GEMM, read per launch: tests switch it between calls
   const char *fe = getenv("QPH_GEMM");
   const int f = fe ? atoi(fe) : 0;
-  return f == 1 || f == 2 ? f : 0;
+  return f >= 1 && f <= 3 ? f : 0;
 }
 static int gemm_cus() {
   if (const char *e = getenv("QPH_GEMM_CUS")) return std::max(1, atoi(e));   // test hook: the choice for another CU count
@@ -919,6 +924,18 @@ static int gemm_row_tiles(const GemmArgs &a, bool big) {
   int t = 0;
   for (int s = 0; s < a.nseg && s < kGemmMaxSeg; s++) t += (a.seg[s].rows + rt - 1) / rt;
   return t;
+}
+// The few-token kernel against the 128-row tiles: a round of those takes ~1.35 us per 128-column block whatever part of
+// it is filled (4096 x 14336 at 16 .. 128 tokens 126 .. 156 us, 14336 x 4096 pairs 48 .. 55, 6144 x 4096 39 .. 42).  The
+// lines that follow from it: 6144 x 4096 and 4096 x 14336 from 512 tokens to the tiles (512: 69 against 46 us, 149 against
+// 156), 4096 x 4096 from 384, gate / up pairs of 14336 x 4096 from 48 (40: 46 against 51 us; 77: 69 against 53)
+bool gemm_wants_tiles(const GemmArgs &a) {
+  if (a.kind != MK_Q8 || a.ntok <= 0 || a.cols % kQB) return false;
+  if (const int f = gemm_forced()) return f == 3;
+  const bool big = gemm_uses_32x32(a);
+  const long wgs = (long)gemm_row_tiles(a, big) * ((a.ntok + kGN - 1) / kGN);
+  int rt, ntt;
+  return skinny_cost(a, gemm_cus(), &rt, &ntt) < 5 + gemm_rounds(wgs) * (big ? kG2Cost : 1.0) * 1.35 * (a.cols / kQB);
 }
 bool gemm_uses_32x32(const GemmArgs &a) {
   return a.kind == MK_Q8 && a.xbt && a.ntok > 0 && gemm_use_32x32(gemm_row_tiles(a, true), (a.ntok + kG2N - 1) / kG2N);
@@ -949,8 +966,17 @@ hipError_t launch_gemm(const GemmArgs &a0, hipStream_t st) {
   if (a.cols % kQB || a.rows <= 0 || a.ldq % 16 || a.ldq < a.cols || a.ldb < a.cols / kQB) return hipErrorInvalidValue;
   const dim3 grid((a.ntok + (big ? kG2N : kGN) - 1) / (big ? kG2N : kGN), tiles);
   if (a.w2 && (a.kind != MK_Q8 || !a.scale2 || !a.wsum2 || a.resid || a.bias || a.gate)) return hipErrorInvalidValue;
+  if (a.kind == MK_Q8 && a.th) {
+    if (!a.tl || a.oh || a.gate) return hipErrorInvalidValue;
+    int rt, ntt;
+    (void)skinny_cost(a, gemm_cus(), &rt, &ntt);
+    if (const char *e = getenv("QPH_SKINNY")) {   // test hook: the tile (two digits, row tiles and token tiles)
+      rt = a.w2 ? 2 : std::max(1, std::min(2, atoi(e) / 10)); ntt = std::max(1, std::min(4, atoi(e) % 10));
+    }
+    return launch_skinny(a, rt, ntt, gemm_cus(), st);
+  }
   if (a.kind == MK_Q8) {
-    if (!a.wsum) return hipErrorInvalidValue;
+    if (!a.wsum || !a.xh || !a.xl) return hipErrorInvalidValue;
     if (big && (!a.xbt || a.ldbt % 4 || a.ldbt < a.ntok)) return hipErrorInvalidValue;
     // a segment launch whose 32 x 32 grid would end in a part-filled round: its first segments on the 32 x 32 kernel,
     // the rest on the 16 x 16 one, when that takes fewer rounds (C4 q / k / v: q alone fills one 32 x 32 round, k + v
@@ -1241,7 +1267,7 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
       a.ob[(size_t)t * a.ldb + head] = bs;
       a.obt[(size_t)head * a.ldbt + t] = bs;
     }
-    int8_t *oh = a.oh + (size_t)t * a.ldo + head * HD, *ol = a.ol + (size_t)t * a.ldo + head * HD;
+    const size_t orow = a.tiled ? (size_t)(t & ~15) * a.ldo + (size_t)head * 2048 + 16 * (t & 15) : (size_t)t * a.ldo + head * HD;
 #pragma unroll
     for (int d = 0; d < DT; d++) {
       uint32_t hh = 0, ll = 0;
@@ -1251,8 +1277,9 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
         hh |= (uint32_t)((q >> 8) & 0xff) << (8 * i);
         ll |= (uint32_t)((q & 0xff) ^ 0x80) << (8 * i);
       }
-      *(uint32_t *)(oh + 16 * d + 4 * lg) = hh;
-      *(uint32_t *)(ol + 16 * d + 4 * lg) = ll;
+      const size_t o = orow + (a.tiled ? 1024 * (d & 1) + 256 * (d >> 1) : 16 * d) + 4 * lg;
+      *(uint32_t *)(a.oh + o) = hh;
+      *(uint32_t *)(a.ol + o) = ll;
     }
     return;
   }

@@ -106,6 +106,27 @@ def test_matmul_q8_rows_equal_decode_arithmetic(rows, cols, B, kernel, monkeypat
         np.testing.assert_array_equal(Y[b], O.rows_q8(q, s, xq, bs), err_msg=f"token {b}")
 
 
+@pytest.mark.parametrize("rows,cols,B", [(7, 128, 1), (16, 1024, 16), (33, 1152, 17), (130, 896, 33), (4113, 2048, 50), (300, 14336, 77),
+                                         (48, 4864, 129), (2100, 512, 700)])
+@pytest.mark.parametrize("tile", ["11", "12", "13", "14", "21", "22", "23", "24"])
+def test_matmul_q8_few_tokens(rows, cols, B, tile, monkeypatch):
+    """the few-token product (K split over the waves), each of its tiles (16 or 32 rows x 16 .. 64 tokens) forced: every
+    token's row bit-identical to rows_q8; row and token counts around the tile edges, column counts that end a round of
+    eight blocks early (1, 7, 9, 38, 112 blocks), more row tiles than workgroups, more token tiles than CUs / 8"""
+    monkeypatch.setenv("QPH_GEMM", "3")
+    monkeypatch.setenv("QPH_SKINNY", tile)
+    rng = np.random.default_rng(rows * 23 + cols + B)
+    q, s = q8_matrix(rng, rows, cols)
+    X = np.stack([act_vector(rng, cols) * rng.uniform(0.1, 10) for _ in range(B)]).astype(np.float32) if cols > 256 else \
+        rng.normal(0, 1, (B, cols)).astype(np.float32)
+    X[B // 2] = 0
+    print(f"q8 few-token matmul tile {tile} rows={rows} cols={cols} B={B}", flush=True)
+    Y = qa.kernel_matmul(q, s, X)
+    for b in range(0, B, max(1, B // 60)):
+        xq, bs = O.quant_act(X[b])
+        np.testing.assert_array_equal(Y[b], O.rows_q8(q, s, xq, bs), err_msg=f"token {b}")
+
+
 @pytest.mark.parametrize("rows,cols,B", [(1000, 4096, 200), (257, 896, 129), (300, 18944, 17), (9, 128, 1), (3584, 3584, 64),
                                          (130, 512, 1024)])
 def test_matmul_q4(rows, cols, B):

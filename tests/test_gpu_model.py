@@ -240,6 +240,25 @@ def test_prefill_q8_kernels_agree(cfg, synth, monkeypatch):
         assert out[0][1] == o[1], "cache rows differ between the kernels"
 
 
+@pytest.mark.parametrize("n", [5, 33, 130])
+@pytest.mark.parametrize("cfg", ["mini", "mini128", "mini_odd", "mini_q4m", "c1"])
+def test_prefill_few_token_kernel_agrees(cfg, n, synth, monkeypatch):
+    """prompts whose q8 products all run on the few-token kernel (QPH_GEMM=3: q / k / v segments with bias, wo and down
+    into the residual, the gate / up pair; the attention's quantised output in its token tiles at head dim 128) give the
+    logits and cache rows of the 16 x 16 kernel (QPH_GEMM=2) bit for bit; mini_q4m mixes it with q4 products"""
+    path = synth(cfg)
+    toks = np.random.default_rng(n).integers(0, qa.CONFIGS[cfg].vocab, n).astype(np.int32)
+    out = []
+    for k in ("2", "3"):
+        monkeypatch.setenv("QPH_GEMM", k)
+        print(f"{cfg}: {n}-token prompt, QPH_GEMM={k}", flush=True)
+        gpu = qa.HipLlama.load(path, max_ctx=n + 3)
+        out.append((gpu.prefill(toks, 1), gpu.snapshot()))
+        gpu.close()
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[0][1] == out[1][1], "cache rows differ between the kernels"
+
+
 def kv_snapshot(k, v):
     """a snapshot in the reference layout (model_llama.cpp:55-63) from per-layer fp16 K / V rows [L][pos][kvd]"""
     pos = k.shape[1]
