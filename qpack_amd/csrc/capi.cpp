@@ -262,7 +262,7 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
     need(q, "q"); need(scale, "scale"); need(X, "X"); need(Y, "Y");
     if (rows <= 0 || B <= 0 || cols <= 0 || cols % 128) throw std::invalid_argument("matmul: rows, B > 0 and cols a positive multiple of 128 required");
     if (kind != QPH_Q8 && kind != QPH_Q4) throw std::invalid_argument("matmul: kind must be QPH_Q8 or QPH_Q4");
-    const int nb = cols / 128, ldb = (nb + 7) / 8 * 8, G = cols / 32, ldg = (G + 3) / 4 * 4;
+    const int nb = cols / 128, ldb = (nb + 7) / 8 * 8, G = cols / 32;
     const size_t qb = kind == QPH_Q8 ? (size_t)rows * cols : (size_t)rows * cols / 2;
     const size_t sb = kind == QPH_Q8 ? 4ull * rows : 2ull * rows * G;
     std::vector<void *> bufs;
@@ -273,19 +273,22 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
       const int ldbt = (B + 63) / 64 * 64;
       float *dxbt = (float *)alloc(4ull * ldbt * nb);
       int8_t *dxh = (int8_t *)alloc((size_t)B * cols), *dxl = (int8_t *)alloc((size_t)B * cols);
-      int *dxg = (int *)alloc(4ull * B * ldg);
       hck(hipMemcpy(dq, q, qb, hipMemcpyHostToDevice), "upload q");
       hck(hipMemcpy(ds, scale, sb, hipMemcpyHostToDevice), "upload scale");
       hck(hipMemcpy(dx, X, 4ull * B * cols, hipMemcpyHostToDevice), "upload X");
       qph::GemmArgs ga{}; ga.kind = kind == QPH_Q8 ? qph::MK_Q8 : qph::MK_Q4; ga.w = (const int8_t *)dq; ga.scale = (const float *)ds;
       ga.rows = rows; ga.cols = cols; ga.xh = dxh; ga.xl = dxl; ga.xb = dxb; ga.ntok = B; ga.ldq = cols; ga.ldb = ldb;
-      ga.xg = dxg; ga.ldg = ldg; ga.y = dy; ga.ldy = rows; ga.xbt = dxbt; ga.ldbt = ldbt;
+      ga.y = dy; ga.ldy = rows; ga.xbt = dxbt; ga.ldbt = ldbt;
       qph::PfQuantArgs qa{}; qa.x = dx; qa.ldx = cols; qa.cols = cols; qa.xh = dxh; qa.xl = dxl; qa.ldq = cols; qa.xb = dxb; qa.ldb = ldb;
-      qa.xg = dxg; qa.ldg = ldg; qa.xbt = dxbt; qa.ldbt = ldbt;
+      qa.xbt = dxbt; qa.ldbt = ldbt;
       if (qph::gemm_wants_tiles(ga)) {   // the few-token kernel: the planes in 16-token tiles
         const size_t tb = (size_t)(B + 15) / 16 * 16 * cols;
         qa.th = (int8_t *)alloc(tb); qa.tl = (int8_t *)alloc(tb); qa.xh = qa.xl = nullptr;
         ga.th = qa.th; ga.tl = qa.tl;
+      }
+      if (kind == QPH_Q4) {
+        qa.fp = (uint16_t *)alloc((size_t)(B + 15) / 16 * 16 * cols * 4);
+        qa.fkind = qph::MK_Q4; ga.fp = qa.fp;
       }
       hck(qph::launch_pf_quant(qph::PRO_QUANT, qa, B, nullptr), "launch quant");
       if (kind == QPH_Q8) {
@@ -293,9 +296,9 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
         hck(qph::launch_rowsum_q8((const int8_t *)dq, rows, cols, dws, nullptr), "launch rowsum");
         ga.wsum = dws;
       } else {
-        int *dns = (int *)alloc(4ull * rows * G); float *dsc = (float *)alloc(4ull * rows * G);
-        hck(qph::launch_q4_prep((const uint8_t *)dq, (const uint16_t *)ds, rows, cols, dns, dsc, nullptr), "launch q4 prep");
-        ga.q4ns = dns; ga.q4sc = dsc;
+        uint16_t *dst = (uint16_t *)alloc(sb);
+        hck(qph::launch_scale_blocks(qph::MK_Q4, (const uint16_t *)ds, rows, cols, dst, nullptr), "launch scale blocks");
+        ga.st = dst;
       }
       hck(qph::launch_gemm(ga, nullptr), "launch gemm");
       hck(hipDeviceSynchronize(), "matmul");

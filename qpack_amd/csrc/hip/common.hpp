@@ -17,11 +17,10 @@ struct DMat {
   const void *q;       // q8: int8 [rows, cols]; q4: u8 [rows, cols / 2]; q1: sign bits u8 [rows, cols / 8]; f32: float
   const void *s;       // q8: f32 [rows]; q4: fp16 [rows, cols / 32]; q1: fp16 [rows, cols / 128]
   int rows, cols, kind;
-  // layer matrices on the batched prompt path: q8 row sums per 128-column block [rows, cols / 128]; q4 nibble sums and
-  // f32 scales per (block, group, row), group-major within each block
+  // layer matrices on the batched prompt path: q8 row sums per 128-column block [rows, cols / 128]; q4 / q1 the scales
+  // block-major (launch_scale_blocks)
   const int *rs;
-  const int *q4ns;
-  const float *q4sc;
+  const uint16_t *st;
 };
 
 // device-resident decode control block: the token to embed, its position, and the greedy output cursor

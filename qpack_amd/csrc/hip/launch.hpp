@@ -177,20 +177,22 @@ struct PfQuantArgs {
   int8_t *xh, *xl; int ldq;
   float *xb; int ldb;
   float *xbt; int ldbt;   // optional: the block scales block-major [cols / 128][ldbt]
-  int *xg; int ldg;   // optional: sum of q per 32-column group [B][ldg] (the q4 product needs it)
   // optional: the planes again in the order the few-token products read them (k_skinny_q8): per 16-token tile (16 ldq
   // bytes apart) the 16-column piece p of each 128-column block (2048 bytes) of token t at byte
   // 1024 (p % 2) + 256 (p / 2) + 16 (t % 16)
   int8_t *th, *tl;
+  // optional: q as two fp16 planes (hi = 256 (q >> 8), lo = q & 255) in the order the q4 / q1 products read them
+  // (k_half), fkind MK_Q4 or MK_Q1: per 16-token tile and 128-column block four 32-column steps x two planes x 1 KiB,
+  // lane 16 lg + t % 16 of step s holding the columns its weight fragment holds
+  uint16_t *fp; int fkind;
 };
 hipError_t launch_pf_quant(int pro, const PfQuantArgs &a, int B, hipStream_t st);
 // Y[t][r] = the row's dot product with token t's quantised activation (+ bias[r]), or Y[t][r] += that when resid.
 //   kind MK_Q8: w int8 [rows][cols], scale f32 [rows], wsum = row sums per 128-column block [rows][ldw] (launch_rowsum_q8)
-//   kind MK_Q4: w packed q4 [rows][cols / 2], q4ns / q4sc = per-group nibble sums and f32 scales, group-major per block
-//               (launch_q4_prep), and the activation's group sums xg [ntok][ldg] (launch_pf_quant)
+//   kind MK_Q4 / MK_Q1: w as stored, the scales block-major in st, the activation's fp16 planes fp
 // one matrix of a multi-matrix product launch (GemmArgs::nseg > 1): its own weights, scales, bias and output
 struct GemmSeg {
-  const int8_t *w; const float *scale; const int *wsum; const int *q4ns; const float *q4sc;
+  const int8_t *w; const float *scale; const int *wsum; const uint16_t *st;
   const float *bias; float *y; int rows, ldy;
 };
 constexpr int kGemmMaxSeg = 3;
@@ -198,17 +200,15 @@ struct GemmArgs {
   int kind;
   const int8_t *w; const float *scale; int rows, cols;
   const int *wsum;   // q8: 128 x the row sums per 128-column block (k_rowsum_q8), [cols / 128][ws_pitch(rows)]
-  const int *q4ns; const float *q4sc;
-  const int *xg; int ldg;
   const int8_t *xh, *xl; const float *xb; int ntok, ldq, ldb;
   const int8_t *th, *tl;   // optional (q8): the planes in 16-token tiles (PfQuantArgs::th), whole tiles allocated
+  // q4 / q1: the activation's fp16 planes (PfQuantArgs::fp), the scales block-major (launch_scale_blocks; st2 of w2)
+  const uint16_t *fp, *st, *st2;
   const float *xbt; int ldbt;   // q8: the block scales again, block-major [cols / 128][ldbt] (ldbt % 4 == 0, >= ntok)
   float *y; int ldy;
   const float *bias;
   int resid;
-  // optional, same layout as y: y = silu(gate) * product (SwiGLU on the up product; gate may be y itself)
-  const float *gate;
-  // optional (q8): a second matrix of the same shape (the up matrix, with w / scale / wsum the gate's): one launch
+  // optional: a second matrix of the same shape (the up matrix, with w / scale / wsum the gate's): one launch
   // computes both products for each 64-row tile and stores only y = silu(gate product) * (up product)
   const int8_t *w2; const float *scale2; const int *wsum2;
   // optional (with w2, 32 x 32 kernel only, rows % 128 == 0): instead of y, the SwiGLU output quantised for the next
@@ -216,7 +216,7 @@ struct GemmArgs {
   // arithmetic: every 128-row tile of the pair is one quantisation block of each token)
   int8_t *oh, *ol; float *ob, *obt;
   // optional: nseg (2 .. kGemmMaxSeg) matrices of this kind and column count over the same activations (q / k / v), the
-  // segment fields replacing w / scale / wsum / q4ns / q4sc / bias / y / ldy / rows; each starts on a fresh row tile
+  // segment fields replacing w / scale / wsum / st / bias / y / ldy / rows; each starts on a fresh row tile
   int nseg;
   GemmSeg seg[kGemmMaxSeg];
   int tile0;   // first row tile of this launch (a launch split over the two q8 kernels; set by launch_gemm)
@@ -228,14 +228,16 @@ size_t gemm_lds_bytes();
 __host__ __device__ inline int ws_pitch(int rows) { return (rows + 63) & ~63; }
 // out[row][block] = sum of W[row] over each 128-column block
 hipError_t launch_rowsum_q8(const int8_t *w, int rows, int cols, int *out, hipStream_t st);
-// q4 rows: per (block, group, row) the sum of the nibbles and the f32 scale, group-major within each 128-column block
-hipError_t launch_q4_prep(const uint8_t *w, const uint16_t *sc, int rows, int cols, int *out_ns, float *out_sc, hipStream_t st);
 // launch_gemm runs a q8 launch with th set on the few-token kernel, others on the tiled ones (which read xh / xl);
 // gemm_wants_tiles: whether th is the faster choice for this product (the pointers need not be set yet)
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t st);
 bool gemm_wants_tiles(const GemmArgs &a);
 // whether launch_gemm runs this q8 launch on the 32 x 32 kernel (the one that can quantise a SwiGLU pair's output)
 bool gemm_uses_32x32(const GemmArgs &a);
+// q4 / q1 products on the f16 matrix cores (skinny.hip): 16 rt rows (8 of each matrix of a pair) x 16 ntt tokens a tile
+hipError_t launch_half(const GemmArgs &a, int cus, hipStream_t st);
+// scales [rows][G] -> [block][row][4] (q4) or [block][row] (q1)
+hipError_t launch_scale_blocks(int kind, const uint16_t *sc, int rows, int cols, uint16_t *out, hipStream_t st);
 // q8 products of few tokens or few rows (skinny.hip): K split over the waves of a workgroup of 16 rt rows (16 of each
 // matrix for a gate / up pair, rt = 2) x 16 ntt tokens; reads the planes from th / tl; ldb a multiple of 8
 hipError_t launch_skinny(const GemmArgs &a, int rt, int ntt, int cus, hipStream_t st);

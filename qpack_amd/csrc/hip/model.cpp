@@ -174,26 +174,20 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
   }
   ctl_ = (Ctl *)dalloc(sizeof(Ctl));
   out_tok_ = (int *)dalloc(4ull * (ctx_ + 1));
-  // batched prompt path: every layer matrix q8 or q4 (the int8 MFMA products; in the default order a model with q1
-  // layers takes its prompts through decode steps); chunks of up to pf_cap_ tokens.  The prompt buffers are allocated
-  // either way: the reference-order prompt (k_ex_gemm, which takes q1 matrices too) uses them
-  pf_ok_ = true;
-  for (const Layer &ly : layers_)
-    for (const DMat *m : {&ly.wq, &ly.wk, &ly.wv, &ly.wo, &ly.wg, &ly.wu, &ly.wd})
-      pf_ok_ = pf_ok_ && (m->kind == MK_Q8 || m->kind == MK_Q4);
+  // batched prompt path, in chunks of up to pf_cap_ tokens; its products' per-matrix data
+  bool half_mats = false;   // some layer matrix is q4 or q1
   {
     for (Layer &ly : layers_)
       for (DMat *m : {&ly.wq, &ly.wk, &ly.wv, &ly.wo, &ly.wg, &ly.wu, &ly.wd}) {
-        if (!pf_ok_) break;   // the batched products' per-matrix sums: q8 / q4 models only
         if (m->kind == MK_Q8) {
           int *rs = (int *)dalloc(4ull * ws_pitch(m->rows) * (m->cols / 128));
           QPH_CK(launch_rowsum_q8((const int8_t *)m->q, m->rows, m->cols, rs, st_));
           m->rs = rs;
         } else {
-          int *ns = (int *)dalloc(4ull * m->rows * (m->cols / 32));
-          float *sc = (float *)dalloc(4ull * m->rows * (m->cols / 32));
-          QPH_CK(launch_q4_prep((const uint8_t *)m->q, (const uint16_t *)m->s, m->rows, m->cols, ns, sc, st_));
-          m->q4ns = ns; m->q4sc = sc;
+          uint16_t *t = (uint16_t *)dalloc(2ull * m->rows * (m->cols / (m->kind == MK_Q4 ? 32 : 128)));
+          QPH_CK(launch_scale_blocks(m->kind, (const uint16_t *)m->s, m->rows, m->cols, t, st_));
+          m->st = t; half_mats = true;
+          pf_q1_ = pf_q1_ || m->kind == MK_Q1;
         }
       }
     QPH_CK(hipStreamSynchronize(st_));
@@ -214,8 +208,7 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
     pf_xbt_ = (float *)dalloc(4ull * pf_ldbt_ * (pf_ldq_ / 128 + 1));
     pf_xb2_ = (float *)dalloc(4 * B * pf_ldb_);
     pf_xbt2_ = (float *)dalloc(4ull * pf_ldbt_ * (pf_ldq_ / 128 + 1));
-    pf_ldg_ = (pf_ldq_ / 32 + 3) / 4 * 4;
-    pf_xg_ = (int *)dalloc(4 * B * pf_ldg_);
+    if (half_mats) pf_fp_ = (uint16_t *)dalloc(4 * B16 * wide);
     pf_tok_ = (int *)dalloc(4 * B);
   }
   // RoPE tables in the reference's precision: inv_i = 1 / theta^(2i/hd) and angle pos * inv_i in double, cos / sin
@@ -504,7 +497,7 @@ void HipLlama::prefill(const int *toks, int n, int want, float *out) {
   for (int i = 0; i < n; i++) if (toks[i] < 0 || toks[i] >= cfg_.vocab) throw std::runtime_error("token id out of range");
   const bool force_steps = getenv("QPH_PREFILL_STEPS") != nullptr;   // test hook: the decode-step path
   // one token (the reference's n == 1 case), or q1 layers in the default order: decode steps
-  if (n == 1 || (!pf_ok_ && !order_) || force_steps) {
+  if (n == 1 || (pf_q1_ && !order_) || force_steps) {
     for (int i = 0; i < n; i++) step(toks[i], i + 1 == n ? want : 0, i + 1 == n ? out : nullptr);
     if (!want) { QPH_CK(hipStreamSynchronize(st_)); check_status(); }
     return;
@@ -536,11 +529,12 @@ void HipLlama::prefill_batched(const int *toks, int n) {
   const int d = cfg_.hidden, ff = cfg_.ffn, nb_ld = pf_ldb_;
   const float eps = cfg_.rms_eps;
   // the products of one activation, first planned (which planes does each read), then quantised for, then launched
-  struct Planes { bool rows, tiles; };
+  struct Planes { bool rows, tiles; int half; };   // half: MK_Q4 or MK_Q1, whose fragments the fp16 planes match
   auto plan = [&](GemmArgs *g, int ng) {
-    Planes p{false, false};
+    Planes p{false, false, 0};
     for (int i = 0; i < ng; i++) {
-      if (gemm_wants_tiles(g[i])) { g[i].th = pf_th_; g[i].tl = pf_tl_; p.tiles = true; }
+      if (g[i].kind != MK_Q8) { if (!p.half) p.half = g[i].kind; }
+      else if (gemm_wants_tiles(g[i])) { g[i].th = pf_th_; g[i].tl = pf_tl_; p.tiles = true; }
       else p.rows = true;
     }
     return p;
@@ -549,18 +543,28 @@ void HipLlama::prefill_batched(const int *toks, int n) {
     PfQuantArgs a{}; a.x = x; a.ldx = ldx; a.norm_w = w; a.eps = eps; a.cols = cols;
     if (p.rows) { a.xh = pf_xh_; a.xl = pf_xl_; }
     if (p.tiles) { a.th = pf_th_; a.tl = pf_tl_; }
-    a.ldq = pf_ldq_; a.xb = pf_xb_; a.ldb = nb_ld; a.xg = pf_xg_; a.ldg = pf_ldg_;
+    if (p.half) { a.fp = pf_fp_; a.fkind = p.half; }
+    a.ldq = pf_ldq_; a.xb = pf_xb_; a.ldb = nb_ld;
     a.xbt = pf_xbt_; a.ldbt = pf_ldbt_;
     QPH_CK(launch_pf_quant(pro, a, B, st_));
   };
+  // quantise, then launch: planes for one of q4 and q1 at a time (a file may mix them among q / k / v)
+  auto products = [&](int pro, const float *x, int ldx, const float *w, int cols, int B, GemmArgs *g, int ng) {
+    Planes p = plan(g, ng);
+    quant(pro, x, ldx, w, cols, B, p);
+    for (int i = 0; i < ng; i++) {
+      if (g[i].kind != MK_Q8 && g[i].kind != p.half) { p = Planes{false, false, g[i].kind}; quant(pro, x, ldx, w, cols, B, p); }
+      QPH_CK(launch_gemm(g[i], st_));
+    }
+  };
   auto operands = [&](int kind, int cols, int B) {
-    GemmArgs a{}; a.kind = kind; a.cols = cols; a.xbt = pf_xbt_; a.ldbt = pf_ldbt_; a.xg = pf_xg_; a.ldg = pf_ldg_;
+    GemmArgs a{}; a.kind = kind; a.cols = cols; a.xbt = pf_xbt_; a.ldbt = pf_ldbt_; a.fp = pf_fp_;
     a.xh = pf_xh_; a.xl = pf_xl_; a.xb = pf_xb_; a.ntok = B; a.ldq = pf_ldq_; a.ldb = nb_ld;
     return a;
   };
-  auto product = [&](const DMat &m, float *y, int ldy, const float *bias, bool resid, int B, const float *gate = nullptr) {
+  auto product = [&](const DMat &m, float *y, int ldy, const float *bias, bool resid, int B) {
     GemmArgs a = operands(m.kind, m.cols, B); a.w = (const int8_t *)m.q; a.scale = (const float *)m.s; a.rows = m.rows;
-    a.wsum = m.rs; a.q4ns = m.q4ns; a.q4sc = m.q4sc; a.y = y; a.ldy = ldy; a.bias = bias; a.resid = resid ? 1 : 0; a.gate = gate;
+    a.wsum = m.rs; a.st = m.st; a.y = y; a.ldy = ldy; a.bias = bias; a.resid = resid ? 1 : 0;
     return a;
   };
   // q / k / v: runs of consecutive matrices of one kind share a launch (q8 files: one launch; q4m: q + k, then v)
@@ -573,11 +577,11 @@ void HipLlama::prefill_batched(const int *toks, int n) {
     for (int i = 0; i < 3;) {
       int j = i + 1;
       while (j < 3 && m[j]->kind == m[i]->kind && m[j]->cols == m[i]->cols) j++;
-      if (j - i == 1 || (m[i]->kind != MK_Q8 && m[i]->kind != MK_Q4)) { g[ng++] = product(*m[i], y[i], ld[i], bias[i], false, B); i++; continue; }
+      if (j - i == 1) { g[ng++] = product(*m[i], y[i], ld[i], bias[i], false, B); i++; continue; }
       GemmArgs a = operands(m[i]->kind, m[i]->cols, B);
       a.nseg = j - i;
       for (int s = i; s < j; s++)
-        a.seg[s - i] = GemmSeg{(const int8_t *)m[s]->q, (const float *)m[s]->s, m[s]->rs, m[s]->q4ns, m[s]->q4sc, bias[s], y[s], m[s]->rows, ld[s]};
+        a.seg[s - i] = GemmSeg{(const int8_t *)m[s]->q, (const float *)m[s]->s, m[s]->rs, m[s]->st, bias[s], y[s], m[s]->rows, ld[s]};
       g[ng++] = a;
       i = j;
     }
@@ -594,8 +598,7 @@ void HipLlama::prefill_batched(const int *toks, int n) {
       uint16_t *kc = kc_ + (size_t)l * ctx_ * kvd_, *vc = vc_ + (size_t)l * ctx_ * kvd_;
       GemmArgs g[3];
       int ng = qkv(ly, B, g);
-      quant(PRO_NORM, pf_x_, d, ly.an, d, B, plan(g, ng));
-      for (int i = 0; i < ng; i++) QPH_CK(launch_gemm(g[i], st_));
+      products(PRO_NORM, pf_x_, d, ly.an, d, B, g, ng);
       // q's RoPE happens in the attention kernel; at head dim 128 (one head = one quantisation block) that kernel also
       // quantises its output for a q8 wo
       PfRopeArgs r{}; r.q = pf_q_; r.ldq = qd_; r.k = pf_k_; r.v = pf_v_; r.ldk = kvd_; r.cos_t = cos_; r.sin_t = sin_;
@@ -614,23 +617,17 @@ void HipLlama::prefill_batched(const int *toks, int n) {
       QPH_CK(launch_pf_attn(t, st_));
       if (!att_q) quant(PRO_QUANT, pf_att_, qd_, nullptr, qd_, B, pl);
       QPH_CK(launch_gemm(g[0], st_));
-      bool fused = false;   // h = silu(gate) * up quantised by the product's store, straight into the second planes
-      if (ly.wg.kind == MK_Q8 && ly.wu.kind == MK_Q8) {   // gate and up in one launch, only h = silu(gate) * up stored
-        GemmArgs &a = g[0];
-        a = product(ly.wg, pf_g_, ff, nullptr, false, B);
-        a.w2 = (const int8_t *)ly.wu.q; a.scale2 = (const float *)ly.wu.s; a.wsum2 = ly.wu.rs;
-        pl = plan(&a, 1);
-        quant(PRO_NORM, pf_x_, d, ly.fn, d, B, pl);
-        fused = !(unfused & 4) && ly.wd.kind == MK_Q8 && ff % 128 == 0 && !pl.tiles && gemm_uses_32x32(a) &&
-                !gemm_wants_tiles(product(ly.wd, pf_x_, d, nullptr, true, B));
-        if (fused) { a.oh = pf_xh2_; a.ol = pf_xl2_; a.ob = pf_xb2_; a.obt = pf_xbt2_; }
-        QPH_CK(launch_gemm(a, st_));
-      } else {
-        g[0] = product(ly.wg, pf_g_, ff, nullptr, false, B);
-        g[1] = product(ly.wu, pf_g_, ff, nullptr, false, B, pf_g_);   // h = silu(gate) * up, in place over the gate product
-        quant(PRO_NORM, pf_x_, d, ly.fn, d, B, plan(g, 2));
-        for (int i = 0; i < 2; i++) QPH_CK(launch_gemm(g[i], st_));
-      }
+      // gate and up in one launch, only h = silu(gate) * up stored; fused: quantised by the product's store, straight into
+      // the second planes
+      GemmArgs &gu = g[0];
+      gu = product(ly.wg, pf_g_, ff, nullptr, false, B);
+      gu.w2 = (const int8_t *)ly.wu.q; gu.scale2 = (const float *)ly.wu.s; gu.wsum2 = ly.wu.rs; gu.st2 = ly.wu.st;
+      pl = plan(&gu, 1);
+      quant(PRO_NORM, pf_x_, d, ly.fn, d, B, pl);
+      const bool fused = !(unfused & 4) && ly.wg.kind == MK_Q8 && ly.wd.kind == MK_Q8 && ff % 128 == 0 && !pl.tiles &&
+                         gemm_uses_32x32(gu) && !gemm_wants_tiles(product(ly.wd, pf_x_, d, nullptr, true, B));
+      if (fused) { gu.oh = pf_xh2_; gu.ol = pf_xl2_; gu.ob = pf_xb2_; gu.obt = pf_xbt2_; }
+      QPH_CK(launch_gemm(gu, st_));
       g[0] = product(ly.wd, pf_x_, d, nullptr, true, B);
       if (fused) {
         g[0].xh = pf_xh2_; g[0].xl = pf_xl2_; g[0].xb = pf_xb2_; g[0].xbt = pf_xbt2_;

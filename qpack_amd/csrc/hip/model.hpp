@@ -139,10 +139,10 @@ class HipLlama {
   void ex_enqueue_head();
   void ex_prefill(const int *toks, int n);
   void enqueue_step(int parts);
-  // batched prompt path (layer matrices q8 / q4)
+  // batched prompt path
+  bool pf_q1_ = false;   // some layer matrix is q1
   static constexpr int kPfChunk = 2048;
-  bool pf_ok_ = false;
-  int pf_cap_ = 0, pf_ldq_ = 0, pf_ldg_ = 0;
+  int pf_cap_ = 0, pf_ldq_ = 0;
   float *pf_x_ = nullptr, *pf_q_ = nullptr, *pf_k_ = nullptr, *pf_v_ = nullptr, *pf_att_ = nullptr, *pf_g_ = nullptr;
   float *pf_xb_ = nullptr, *pf_xbt_ = nullptr;   // block scales token-major [B][nb], block-major [nb][pf_ldbt_]
   int pf_ldbt_ = 0;
@@ -151,7 +151,8 @@ class HipLlama {
   int pf_ldb_ = 0;                               // row pitch of the block scales
   int8_t *pf_xh2_ = nullptr, *pf_xl2_ = nullptr;   // second planes: the SwiGLU output quantised by the gate / up store
   float *pf_xb2_ = nullptr, *pf_xbt2_ = nullptr;
-  int *pf_tok_ = nullptr, *pf_xg_ = nullptr;
+  uint16_t *pf_fp_ = nullptr;   // fp16 planes (PfQuantArgs::fp), for models with q4 or q1 layers
+  int *pf_tok_ = nullptr;
   void prefill_batched(const int *toks, int n);
 
   void *dalloc(size_t bytes);

@@ -8,6 +8,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "act.hpp"
 #include "launch.hpp"
@@ -291,6 +292,347 @@ hipError_t launch_skinny(const GemmArgs &a, int rt, int ntt, int cus, hipStream_
 #define QPH_SK(R, N) if (rt == R && ntt == N) return launch_skinny_t<R, N, kSkDepth, kSkDepth>(a, nrt, cus, st);
   QPH_SK(1, 1) QPH_SK(1, 2) QPH_SK(1, 3) QPH_SK(1, 4) QPH_SK(2, 1) QPH_SK(2, 2) QPH_SK(2, 3) QPH_SK(2, 4)
 #undef QPH_SK
+  return hipErrorInvalidValue;
+}
+
+// ------------------------------------------------------------------ q4 and q1 weights on the f16 matrix cores
+// A q4 group (32 columns) is a dot product of 4-bit integers with 16-bit ones: at most 8 x 32 x 32767 < 2^23 in size, so
+// v_mfma_f32_16x16x32_f16 gives it exactly, as a float: the weights n = nibble - 8 are exact halves, the activation goes in
+// as two halves q = hi + lo (hi = 256 (q >> 8), lo = q & 255), every product and partial sum is an integer below 2^24.
+// What is left for the vector ALU is one fma per output and group, with the group's fp16 scale; on the int8 cores it is a
+// shift-add, a conversion and an fma, and the offset corrections.  A q1 group (128 columns) is below 2^22 likewise.
+//   blk = sum over the block's groups of scale * sum, acc = fma(bs[token][block], blk, acc)
+// Tile: 16 RT rows x 16 NTT tokens per workgroup; its 8 waves take every eighth block each, add no barrier until the tile's
+// end, and their fp32 partials are summed there in wave order through LDS.
+// Operands: weights from HBM to registers as stored.  q4: lane l loads the 16 bytes of group l / 16 of row l % 16; a 4 x 4
+// transpose of dwords over the four 16-lane rows (permlane swaps) gives every lane dword l / 16 of each group, and a dword
+// becomes four half pairs with a mask, 0x6400 (1024 + nibble) and one packed subtraction.  q1: dword l / 16 of the block; a
+// shift and a bit-field insert turn two bits into +-1.  Activations in the order these fragments have (PfQuantArgs::fp: 1
+// KiB of consecutive bytes each), straight from L2 to registers, one block ahead (64 rows by 48 tokens, or 32 by 64, spill
+// with q4: 2 to 4 times slower).  The rows' scales of a block (512 bytes,
+// one load) are handed to the lanes through LDS, the tokens' block scales stay in LDS from the start.
+// Measured (MI355X, weights from HBM, us; before: 128 x 128 tiles on the int8 cores): q4 3584 x 18944 at 150 tokens 780 ->
+// 99, 18944 x 3584 255 -> 71, 896 x 4864 at 512 tokens 164 -> 20.  A block of a 64 x 32 tile is 64 MFMAs and ~330 vector
+// instructions per wave; without any loads 150 tokens of 18944 x 3584 take 9 % less: their issue bounds it, ahead of L2.
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef float f4v __attribute__((ext_vector_type(4)));
+
+// lane l of dword j: group l / 16's dword j -> dword l / 16 of group j
+__device__ __forceinline__ void transpose4(uint32_t &a, uint32_t &b, uint32_t &c, uint32_t &d) {
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1\n\t"
+               "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1"
+               : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+}
+// halves (b0.lo, b2.lo, b0.hi, b2.hi, b1.lo, b3.lo, b1.hi, b3.hi) of the dword's four bytes, each nibble - 8.  A nibble in
+// mantissa bits 0-3 under the exponent of 1024 is 1024 + n, in bits 4-7 under that of 64 it is 64 + n: exact halves, so is
+// the difference.  c1 / c2 (0x64006400 / 0x54005400) come in registers: v_and_or_b32 takes one constant besides
+__device__ __forceinline__ h8v q4_half8(uint32_t w, uint32_t c1, uint32_t c2) {
+  const uint32_t v = w >> 8;
+  const h2v o1 = {(_Float16)1032, (_Float16)1032}, o2 = {(_Float16)72, (_Float16)72};
+  auto bits = [](h2v x) { return __builtin_bit_cast(uint32_t, x); };
+  const uint32_t p0 = bits(__builtin_bit_cast(h2v, (w & 0x000f000fu) | c1) - o1);
+  const uint32_t p1 = bits(__builtin_bit_cast(h2v, (w & 0x00f000f0u) | c2) - o2);
+  const uint32_t p2 = bits(__builtin_bit_cast(h2v, (v & 0x000f000fu) | c1) - o1);
+  const uint32_t p3 = bits(__builtin_bit_cast(h2v, (v & 0x00f000f0u) | c2) - o2);
+  return __builtin_bit_cast(h8v, make_uint4(p0, p1, p2, p3));
+}
+// step s of a q1 dword: halves (bit 4 s + j, bit 16 + 4 s + j), j = 0..3, as -1 (set) or +1
+__device__ __forceinline__ h8v q1_half8(uint32_t w, int s) {
+  uint32_t p[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) p[j] = ((w << (15 - 4 * s - j)) & 0x80008000u) | 0x3c003c00u;
+  return __builtin_bit_cast(h8v, make_uint4(p[0], p[1], p[2], p[3]));
+}
+
+template <int KIND, int RT, int NTT>
+__global__ __launch_bounds__(kSkWaves * 64) void k_half(GemmArgs a, int nrt, int ntk, int tg, int rg) {
+  constexpr bool Q4 = KIND == MK_Q4;
+  constexpr int RW = 16 * RT, NT = 16 * NTT, P = RW + 4, SB = Q4 ? 8 : 2;   // SB: scale bytes per row and block
+  extern __shared__ __align__(16) char hsm[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+  const int nb = a.cols / kQB;
+  float *red = (float *)hsm;                                  // [8 waves][NT][P] partials
+  char *scl = hsm + (size_t)kSkWaves * NT * P * 4 + wave * (RW * SB);   // this wave's block scales [RW][SB]
+  float *bsl = (float *)(hsm + (size_t)kSkWaves * (NT * P * 4 + RW * SB));   // [nb][NT]
+  const bool paired = a.w2 != nullptr;   // the tile's first RW / 2 rows from the gate matrix, the others the same rows of up
+  // token tile tk and row tiles rt0, rt0 + rts, ...: the XCD's workgroups are dealt in sets of tg token tiles x rg row tiles
+  const int q = (int)blockIdx.x >> 3, in_set = q % (tg * rg);
+  const int rts = 8 * rg, rt0 = in_set / tg * 8 + (blockIdx.x & 7), tk = q / (tg * rg) * tg + in_set % tg;
+  const int mine = rt0 < nrt && tk < ntk ? (nrt - rt0 + rts - 1) / rts : 0;
+  if (!mine) return;
+  const int rowb = Q4 ? a.cols / 2 : a.cols / 8, blkb = Q4 ? 64 : 16;   // bytes per row, per row and block
+
+  struct Tile { const uint8_t *w, *w2; const uint16_t *st, *st2; const float *bias; float *y; int rows, ldy, r0; };
+  auto tile_of = [&](int rt) {
+    Tile t{(const uint8_t *)a.w, (const uint8_t *)a.w2, a.st, a.st2, a.bias, a.y, a.rows, a.ldy, rt * (paired ? RW / 2 : RW)};
+    if (a.nseg > 1) {
+      int base = 0;
+      bool found = false;
+#pragma unroll
+      for (int s = 0; s < kGemmMaxSeg; s++)
+        if (!found && s < a.nseg) {
+          const GemmSeg &g = a.seg[s];
+          const int n = (g.rows + RW - 1) / RW;
+          if (rt < base + n || s == a.nseg - 1) {
+            t = Tile{(const uint8_t *)g.w, nullptr, g.st, nullptr, g.bias, g.y, g.rows, g.ldy, (rt - base) * RW};
+            found = true;
+          }
+          base += n;
+        }
+    }
+    return t;
+  };
+
+  // the tokens' block scales
+  for (int i = tid; i < nb * NT; i += kSkWaves * 64) {
+    const int b = i / NT, t = tk * NT + i % NT;
+    bsl[i] = a.xb[(size_t)min(t, a.ntok - 1) * a.ldb + b];
+  }
+
+  // this wave's stream: blocks wave, wave + 8, ... of each of its row tiles
+  const int nj = wave < nb ? (nb - wave + kSkWaves - 1) / kSkWaves : 0;
+  int ltile = 0, lj = 0;   // the next weights to load
+  const uint8_t *wrow[RT];
+  const char *srow;
+  size_t sstep = 0;
+  auto w_tile = [&]() {
+    const Tile t = tile_of(rt0 + ltile * rts);
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+      const bool up = paired && i >= RT / 2;
+      const int row = min(t.r0 + 16 * (up ? i - RT / 2 : i) + lr, t.rows - 1);
+      wrow[i] = (up ? t.w2 : t.w) + (size_t)row * rowb + (Q4 ? 16 : 4) * lg;
+    }
+    const int l = lane & (RW - 1);
+    const bool up = paired && l >= RW / 2;
+    srow = (const char *)(up ? t.st2 : t.st) + (size_t)min(t.r0 + (up ? l - RW / 2 : l), t.rows - 1) * SB;
+    sstep = (size_t)t.rows * SB;
+  };
+  typedef typename std::conditional<Q4, uint4, uint32_t>::type raw_t;
+  typedef typename std::conditional<Q4, uint2, uint16_t>::type scr_t;
+  auto load_w = [&](raw_t (&A)[RT], scr_t &S) {
+    const int b = min(wave + kSkWaves * lj, nb - 1);
+#pragma unroll
+    for (int i = 0; i < RT; i++) A[i] = *(const raw_t *)(wrow[i] + (size_t)b * blkb);
+    S = *(const scr_t *)(srow + (size_t)b * sstep);
+    if (lj + 1 < nj) lj++;
+    else if (ltile + 1 < mine) { lj = 0; ltile++; w_tile(); }
+  };
+  const int nt16 = (a.ntok + 15) / 16;
+  const char *fb[NTT];
+#pragma unroll
+  for (int n = 0; n < NTT; n++) fb[n] = (const char *)a.fp + (size_t)min(tk * NTT + n, nt16 - 1) * nb * 8192 + 16 * lane;
+  int bj = 0;
+  h8v B[4][NTT][2];
+  auto load_b = [&](int s) {
+    const size_t o = (size_t)min(wave + kSkWaves * bj, nb - 1) * 8192 + 2048 * s;
+#pragma unroll
+    for (int n = 0; n < NTT; n++)
+#pragma unroll
+      for (int pl = 0; pl < 2; pl++) B[s][n][pl] = *(const h8v *)(fb[n] + o + 1024 * pl);
+  };
+
+  f4v acc[RT][NTT];
+  auto zero = [&]() {
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+      for (int n = 0; n < NTT; n++) acc[i][n] = (f4v){0.f, 0.f, 0.f, 0.f};
+  };
+  zero();
+  raw_t A[RT];
+  scr_t S;
+  uint32_t c1 = 0x64006400u, c2 = 0x54005400u;
+  asm volatile("" : "+v"(c1), "+v"(c2));
+  w_tile();
+  load_w(A, S);
+#pragma unroll
+  for (int s = 0; s < 4; s++) load_b(s);
+  bj = nj > 1 ? 1 : 0;
+  __syncthreads();   // the block scales
+
+  auto block = [&](int b) {
+    // this block's row scales to the lanes that hold the rows (LDS operations of a wave complete in order)
+    if (RW == 64 || lane < RW) *(scr_t *)(scl + (lane & (RW - 1)) * SB) = S;
+    uint32_t q[RT][4];
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+      if constexpr (Q4) {
+        q[i][0] = A[i].x; q[i][1] = A[i].y; q[i][2] = A[i].z; q[i][3] = A[i].w;
+        transpose4(q[i][0], q[i][1], q[i][2], q[i][3]);
+      } else {
+        q[i][0] = A[i];
+      }
+    }
+    load_w(A, S);   // the next block's
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    h4v sc[RT][4];   // q4: row i's four groups; q1: [0] the four rows
+#pragma unroll
+    for (int i = 0; i < RT; i++) {
+      if (Q4) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          const h8v v = *(const h8v *)(scl + (16 * i + 4 * lg + 2 * k) * SB);
+          sc[i][2 * k] = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+          sc[i][2 * k + 1] = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+        }
+      } else {
+        sc[i][0] = *(const h4v *)(scl + (16 * i + 4 * lg) * SB);
+      }
+    }
+    float bs[NTT];
+#pragma unroll
+    for (int n = 0; n < NTT; n++) bs[n] = bsl[b * NT + 16 * n + lr];
+    f4v blk[RT][NTT];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      h8v F[RT];
+#pragma unroll
+      for (int i = 0; i < RT; i++) F[i] = Q4 ? q4_half8(q[i][s], c1, c2) : q1_half8(q[i][0], s);
+#pragma unroll
+      for (int n = 0; n < NTT; n++)
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+          f4v T = (f4v){0.f, 0.f, 0.f, 0.f};
+          if (!Q4 && s > 0) T = blk[i][n];   // q1: one sum for the block
+          T = __builtin_amdgcn_mfma_f32_16x16x32_f16(F[i], B[s][n][0], T, 0, 0, 0);
+          T = __builtin_amdgcn_mfma_f32_16x16x32_f16(F[i], B[s][n][1], T, 0, 0, 0);
+          if (!Q4) { blk[i][n] = T; continue; }
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float w = (float)sc[i][r][s];
+            blk[i][n][r] = s == 0 ? w * T[r] : __builtin_fmaf(w, T[r], blk[i][n][r]);
+          }
+        }
+      load_b(s);
+    }
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+      for (int n = 0; n < NTT; n++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float v = Q4 ? blk[i][n][r] : -(float)sc[i][0][r] * blk[i][n][r];
+          acc[i][n][r] = __builtin_fmaf(bs[n], v, acc[i][n][r]);
+        }
+    bj = bj + 1 < nj ? bj + 1 : 0;
+  };
+
+  for (int tile = 0; tile < mine; tile++) {
+    for (int j = 0; j < nj; j++) block(wave + kSkWaves * j);
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+      for (int n = 0; n < NTT; n++)
+        *(f4v *)(red + (wave * NT + 16 * n + lr) * P + 16 * i + 4 * lg) = acc[i][n];
+    zero();
+    lds_barrier();
+    const Tile t = tile_of(rt0 + tile * rts);
+    auto sum = [&](int tok, int row) {
+      f4v v = *(const f4v *)(red + tok * P + row);
+#pragma unroll
+      for (int w = 1; w < kSkWaves; w++) v += *(const f4v *)(red + (w * NT + tok) * P + row);
+      return v;
+    };
+    const int quads = paired ? RW / 8 : RW / 4;
+    for (int e = tid; e < NT * quads; e += kSkWaves * 64) {
+      const int tok = e / quads, cq = e % quads, gt = tk * NT + tok, row = t.r0 + 4 * cq;
+      if (gt >= a.ntok) continue;
+      f4v v = sum(tok, 4 * cq);
+      float *yt = t.y + (size_t)gt * t.ldy;
+      if (paired) {
+        const f4v u = sum(tok, RW / 2 + 4 * cq);
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = sk_silu_mul(v[r], u[r]);
+      }
+      if (row + 3 < t.rows && (t.ldy & 3) == 0) {
+        if (a.resid) v += *(const f4v *)(yt + row);
+        else if (t.bias) v += *(const f4v *)(t.bias + row);
+        *(f4v *)(yt + row) = v;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (row + r < t.rows) yt[row + r] = a.resid ? yt[row + r] + v[r] : t.bias ? v[r] + t.bias[row + r] : v[r];
+      }
+    }
+    lds_barrier();
+  }
+}
+
+// scales of a q4 / q1 matrix [rows][G] -> block-major: out[block][row][4] (q4) or out[block][row] (q1)
+__global__ __launch_bounds__(256) void k_scale_blocks(const uint16_t *sc, int rows, int G, int per, uint16_t *out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)rows * G) return;
+  const int r = (int)(i / G), g = (int)(i % G);
+  out[((size_t)(g / per) * rows + r) * per + g % per] = sc[i];
+}
+hipError_t launch_scale_blocks(int kind, const uint16_t *sc, int rows, int cols, uint16_t *out, hipStream_t st) {
+  if (cols % kQB || rows <= 0 || (kind != MK_Q4 && kind != MK_Q1)) return hipErrorInvalidValue;
+  const int per = kind == MK_Q4 ? 4 : 1, G = cols / kQB * per;
+  const int64_t n = (int64_t)rows * G;
+  hipLaunchKernelGGL(k_scale_blocks, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, sc, rows, G, per, out);
+  return hipGetLastError();
+}
+
+// token tiles in sets of tg: the workgroups on the chip at a time share a set's activations, which then stay in the XCDs'
+// L2 while the weights stream past (18944 x 3584, 2048 tokens: one set of 64 tiles 1194 us, sets of 16 / 8 / 4 / 2
+// 919 / 865 / 861 / 910; up to 16 tiles one set is as fast)
+static void half_sets(int ntk, int *sets, int *tg) {
+  const int cap = ntk <= 16 ? 16 : 8;
+  *sets = (ntk + cap - 1) / cap; *tg = (ntk + *sets - 1) / *sets;
+}
+static size_t half_lds(int kind, int rt, int ntt, int nb) {
+  return (size_t)kSkWaves * (16 * ntt * (16 * rt + 4) * 4 + 16 * rt * (kind == MK_Q4 ? 8 : 2)) + (size_t)nb * 16 * ntt * 4;
+}
+static int half_row_tiles(const GemmArgs &a, int rt) {
+  const int rw = a.w2 ? 8 * rt : 16 * rt;
+  if (a.nseg < 2) return (a.rows + rw - 1) / rw;
+  int n = 0;
+  for (int s = 0; s < a.nseg; s++) n += (a.seg[s].rows + rw - 1) / rw;
+  return n;
+}
+template <int KIND, int RT, int NTT>
+static hipError_t launch_half_t(const GemmArgs &a, int cus, hipStream_t st) {
+  const int nrt = half_row_tiles(a, RT), nt16 = (a.ntok + 15) / 16, ntk = (nt16 + NTT - 1) / NTT;
+  int sets, tg;
+  half_sets(ntk, &sets, &tg);
+  const int per = sk_tiles_per_wg(nrt, tg, cus), rg = ((nrt + 7) / 8 + per - 1) / per;
+  const size_t lds = half_lds(KIND, RT, NTT, a.cols / kQB);
+  if (lds > 160 * 1024) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_half<KIND, RT, NTT>), dim3((unsigned)(8 * sets * tg * rg)), dim3(kSkWaves * 64), lds, st, a, nrt, ntk, tg, rg);
+  return hipGetLastError();
+}
+// The tile shape for a launch: a start of ~5 us, then per row tile of a workgroup every wave's blocks and ~1 us for its
+// end (block times with every CU busy, from the shapes above).  32-row tiles where 64-row ones leave CUs idle.
+static void half_tile(const GemmArgs &a, int cus, int *rt, int *ntt) {
+  static const int shape[4][2] = {{2, 1}, {2, 2}, {4, 1}, {4, 2}};
+  static const double block_us[4] = {1.55, 2.0, 2.1, 2.45};
+  const int rounds = (a.cols / kQB + kSkWaves - 1) / kSkWaves, nt16 = (a.ntok + 15) / 16;
+  double best = 1e30;
+  for (int i = 0; i < 4; i++) {
+    const int ntk = (nt16 + shape[i][1] - 1) / shape[i][1];
+    int sets, tg;
+    half_sets(ntk, &sets, &tg);
+    const double c = sets * sk_tiles_per_wg(half_row_tiles(a, shape[i][0]), tg, cus) * (rounds * block_us[i] + 1);
+    if (c < best) { best = c; *rt = shape[i][0]; *ntt = shape[i][1]; }
+  }
+}
+hipError_t launch_half(const GemmArgs &a, int cus, hipStream_t st) {
+  if ((a.kind != MK_Q4 && a.kind != MK_Q1) || !a.fp || a.ldb < a.cols / kQB || (a.w2 && !a.st2)) return hipErrorInvalidValue;
+  int rt, ntt;
+  half_tile(a, cus, &rt, &ntt);
+  if (const char *e = getenv("QPH_SKINNY")) {   // test hook: the tile (two digits, rows / 16 and tokens / 16)
+    rt = atoi(e) / 10 >= 4 ? 4 : 2; ntt = std::max(1, std::min(2, atoi(e) % 10));
+  }
+#define QPH_HF(R, N)                                                      \
+  if (rt == R && ntt == N)                                                \
+    return a.kind == MK_Q4 ? launch_half_t<MK_Q4, R, N>(a, cus, st) : launch_half_t<MK_Q1, R, N>(a, cus, st);
+  QPH_HF(2, 1) QPH_HF(2, 2) QPH_HF(4, 1) QPH_HF(4, 2)
+#undef QPH_HF
   return hipErrorInvalidValue;
 }
 

@@ -150,6 +150,35 @@ def test_matmul_q4(rows, cols, B):
         assert np.all(np.abs(Y[b] - y_o) <= 2e-6 * mag + 1e-30), (b, float(np.max(np.abs(Y[b] - y_o) / (mag + 1e-30))))
 
 
+@pytest.mark.parametrize("rows,cols,B", [(7, 128, 1), (31, 1024, 16), (33, 1152, 17), (65, 896, 33), (4113, 2048, 50), (300, 18944, 77),
+                                         (48, 4864, 129), (2100, 512, 700)])
+@pytest.mark.parametrize("tile", ["21", "22", "41", "42"])
+def test_matmul_q4_half_products(rows, cols, B, tile, monkeypatch):
+    """the q4 product on the f16 matrix cores with each of its tiles forced (32 or 64 rows x 16 or 32 tokens): as
+    test_matmul_q4, at row and token counts around the tile edges, column counts that leave some of the eight waves
+    without a block or with one fewer, and more token tiles than one set holds.  Extreme inputs: weights all -8 against
+    activations all at the quantiser's limit (the group sum 32 x 8 x 32767 must come out exact as a float)"""
+    monkeypatch.setenv("QPH_SKINNY", tile)
+    rng = np.random.default_rng(rows * 29 + cols + B)
+    q = rng.integers(0, 256, (rows, cols // 2)).astype(np.uint8)
+    q[0] = 0x00; q[min(1, rows - 1)] = 0xff
+    s = (rng.random((rows, cols // 32)) * 0.01 + 1e-4).astype(np.float16).view(np.uint16)
+    X = rng.normal(0, 1, (B, cols)).astype(np.float32)
+    X[0] = 3.5                                      # every activation 32767
+    X[B // 2] = 0 if B > 1 else X[0]
+    print(f"q4 half product tile {tile} rows={rows} cols={cols} B={B}", flush=True)
+    Y = qa.kernel_matmul(q, s, X)
+    for b in range(0, B, max(1, B // 40)):
+        xq, bs = O.quant_act(X[b])
+        gs = O.group_sums_q4(q, xq)
+        comb = s.view(np.float16).astype(np.float64) * np.repeat(bs, 4)[None, :]
+        mag = np.abs(comb * gs).sum(1)
+        y64 = (comb * gs).sum(1)
+        # fp32: the products rounded twice, at most 4 + ceil(blocks / 8) + 8 additions, 2^-24 each
+        tol = (14 + cols // 1024) * 2.0 ** -24 * mag
+        assert np.all(np.abs(Y[b] - y64) <= tol + 1e-30), (b, float(np.max(np.abs(Y[b] - y64) / (mag + 1e-30))))
+
+
 @pytest.mark.parametrize("kind", ["q8", "q4"])
 @pytest.mark.parametrize("rows,cols,B", [(48, 1024, 6), (257, 896, 64), (300, 4096, 1), (130, 512, 27), (64, 14336, 5),
                                          (1000, 4096, 40)])
