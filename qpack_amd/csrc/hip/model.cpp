@@ -187,7 +187,6 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
           uint16_t *t = (uint16_t *)dalloc(2ull * m->rows * (m->cols / (m->kind == MK_Q4 ? 32 : 128)));
           QPH_CK(launch_scale_blocks(m->kind, (const uint16_t *)m->s, m->rows, m->cols, t, st_));
           m->st = t; half_mats = true;
-          pf_q1_ = pf_q1_ || m->kind == MK_Q1;
         }
       }
     QPH_CK(hipStreamSynchronize(st_));
@@ -496,8 +495,7 @@ void HipLlama::prefill(const int *toks, int n, int want, float *out) {
   if (pos_ + n > ctx_) throw std::runtime_error("context window full (" + std::to_string(ctx_) + " tokens)");
   for (int i = 0; i < n; i++) if (toks[i] < 0 || toks[i] >= cfg_.vocab) throw std::runtime_error("token id out of range");
   const bool force_steps = getenv("QPH_PREFILL_STEPS") != nullptr;   // test hook: the decode-step path
-  // one token (the reference's n == 1 case), or q1 layers in the default order: decode steps
-  if (n == 1 || (pf_q1_ && !order_) || force_steps) {
+  if (n == 1 || force_steps) {   // one token: the reference's n == 1 case
     for (int i = 0; i < n; i++) step(toks[i], i + 1 == n ? want : 0, i + 1 == n ? out : nullptr);
     if (!want) { QPH_CK(hipStreamSynchronize(st_)); check_status(); }
     return;

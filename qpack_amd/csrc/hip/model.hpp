@@ -140,7 +140,6 @@ class HipLlama {
   void ex_prefill(const int *toks, int n);
   void enqueue_step(int parts);
   // batched prompt path
-  bool pf_q1_ = false;   // some layer matrix is q1
   static constexpr int kPfChunk = 2048;
   int pf_cap_ = 0, pf_ldq_ = 0;
   float *pf_x_ = nullptr, *pf_q_ = nullptr, *pf_k_ = nullptr, *pf_v_ = nullptr, *pf_att_ = nullptr, *pf_g_ = nullptr;

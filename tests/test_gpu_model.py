@@ -259,6 +259,39 @@ def test_prefill_few_token_kernel_agrees(cfg, n, synth, monkeypatch):
     assert out[0][1] == out[1][1], "cache rows differ between the kernels"
 
 
+@pytest.mark.parametrize("n", [2, 17, 70, 300])
+@pytest.mark.parametrize("cfg,tile", [("mini_q1", "21"), ("mini_q1", "42"), ("mini_q1m", "22"), ("mini_q1m", "41"), ("mini_q1m", "")])
+def test_batched_prefill_q1(cfg, tile, n, synth, monkeypatch):
+    """prompts of models with q1 MLP matrices go through the batched products (k_half, its tiles forced): logits and every
+    cache row against the oracle's decode steps and against this library's (QPH_PREFILL_STEPS), the greedy continuation
+    against the oracle's up to a near-tie; mini_q1m mixes q1 and q8 down matrices"""
+    if tile:
+        monkeypatch.setenv("QPH_SKINNY", tile)
+    path = synth(cfg)
+    shape = qa.CONFIGS[cfg]
+    kvd = shape.kv_heads * shape.head_dim
+    gpu = qa.HipLlama.load(path, max_ctx=n + 40)
+    orc = O.Oracle(path, max_ctx=n + 40)
+    toks = np.random.default_rng(n).integers(0, shape.vocab, n).astype(np.int32)
+    print(f"{cfg} tile {tile}: {n}-token prompt", flush=True)
+    lg = gpu.prefill(toks, 1)
+    for t in toks:
+        lo = orc.step(int(t), 1)
+    err, ok = close(lg, lo)
+    assert ok, f"logits max|d| {err}"
+    _, kb, vb = split_snapshot(gpu.snapshot(), shape.layers, kvd)
+    ko, vo = orc.kv_cache()
+    for a, b in ((kb, ko[:, :n].view(np.float16)), (vb, vo[:, :n].view(np.float16))):
+        d = np.abs(a.astype(np.float32) - b.astype(np.float32))
+        assert d.max() <= 1e-2 + 2e-3 * np.abs(b.astype(np.float32)).max(), float(d.max())
+    assert_greedy_agrees(gpu, orc, int(np.argmax(lo)), 24, err)
+    gpu.reset()
+    monkeypatch.setenv("QPH_PREFILL_STEPS", "1")
+    err, ok = close(gpu.prefill(toks, 1), lg)
+    assert ok, f"steps against the batched prompt: logits max|d| {err}"
+    gpu.close(); orc.close()
+
+
 def kv_snapshot(k, v):
     """a snapshot in the reference layout (model_llama.cpp:55-63) from per-layer fp16 K / V rows [L][pos][kvd]"""
     pos = k.shape[1]
