@@ -261,6 +261,10 @@ struct PfAttnArgs {
   int ntok, p0, nh, nkv, hd;
   // optional: q not yet rotated - the kernel applies RoPE (k_pf_rope's arithmetic) as it loads q
   const float *cos_t, *sin_t;
+  // optional: part_floats floats of scratch for batches whose workgroups do not fill the chip - the cache is then split
+  // over several workgroups per tile, whose partial outputs a second launch merges
+  float *part; size_t part_floats;
+  int nsplit;   // set by the launcher
   int tiled;   // oh / ol in 16-token tiles (PfQuantArgs::th), not rows
   // optional (hd 128, one head = one 128-column block): the output quantised for the wo product instead of att -
   // planes oh / ol [ntok][ldo], block scales ob [ntok][ldb] and obt [nh][ldbt] (the quantiser's arithmetic)

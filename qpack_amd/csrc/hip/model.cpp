@@ -175,14 +175,14 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
   ctl_ = (Ctl *)dalloc(sizeof(Ctl));
   out_tok_ = (int *)dalloc(4ull * (ctx_ + 1));
   // batched prompt path, in chunks of up to pf_cap_ tokens; its products' per-matrix data
-  bool half_mats = false;   // some layer matrix is q4 or q1
+  bool half_mats = false, q8_mats = false;   // some layer matrix is q4 or q1, some is q8
   {
     for (Layer &ly : layers_)
       for (DMat *m : {&ly.wq, &ly.wk, &ly.wv, &ly.wo, &ly.wg, &ly.wu, &ly.wd}) {
         if (m->kind == MK_Q8) {
           int *rs = (int *)dalloc(4ull * ws_pitch(m->rows) * (m->cols / 128));
           QPH_CK(launch_rowsum_q8((const int8_t *)m->q, m->rows, m->cols, rs, st_));
-          m->rs = rs;
+          m->rs = rs; q8_mats = true;
         } else {
           uint16_t *t = (uint16_t *)dalloc(2ull * m->rows * (m->cols / (m->kind == MK_Q4 ? 32 : 128)));
           QPH_CK(launch_scale_blocks(m->kind, (const uint16_t *)m->s, m->rows, m->cols, t, st_));
@@ -198,9 +198,11 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
     pf_k_ = (float *)dalloc(4 * B * kvd_); pf_v_ = (float *)dalloc(4 * B * kvd_);
     pf_g_ = (float *)dalloc(4 * B * ff);
     pf_xh_ = (int8_t *)dalloc(B * pf_ldq_); pf_xl_ = (int8_t *)dalloc(B * pf_ldq_);
-    pf_xh2_ = (int8_t *)dalloc(B * pf_ldq_); pf_xl2_ = (int8_t *)dalloc(B * pf_ldq_);   // the SwiGLU output, quantised
     const size_t B16 = (B + 15) / 16 * 16;
-    pf_th_ = (int8_t *)dalloc(B16 * pf_ldq_); pf_tl_ = (int8_t *)dalloc(B16 * pf_ldq_);
+    if (q8_mats) {
+      pf_th_ = (int8_t *)dalloc(B16 * pf_ldq_); pf_tl_ = (int8_t *)dalloc(B16 * pf_ldq_);
+      pf_xh2_ = (int8_t *)dalloc(B * pf_ldq_); pf_xl2_ = (int8_t *)dalloc(B * pf_ldq_);   // the SwiGLU output, quantised
+    }
     pf_ldb_ = ((int)wide / 128 + 7) / 8 * 8;   // whole 8-block rounds, 16-byte aligned
     pf_xb_ = (float *)dalloc(4 * B * pf_ldb_);
     pf_ldbt_ = (int)(B + 63) / 64 * 64;
@@ -603,6 +605,7 @@ void HipLlama::prefill_batched(const int *toks, int n) {
       r.kc = kc; r.vc = vc; r.p0 = p0; r.nh = cfg_.heads; r.nkv = cfg_.kv_heads; r.hd = cfg_.head_dim; r.skip_q = !(unfused & 1);
       QPH_CK(launch_pf_rope(r, B, st_));
       PfAttnArgs t{}; t.q = pf_q_; t.ldq = qd_; t.kc = kc; t.vc = vc; t.att = pf_att_; t.lda = qd_;
+      t.part = pf_g_; t.part_floats = (size_t)pf_cap_ * ff;   // free until gate / up
       t.ntok = B; t.p0 = p0; t.nh = cfg_.heads; t.nkv = cfg_.kv_heads; t.hd = cfg_.head_dim;
       if (!(unfused & 1)) { t.cos_t = cos_; t.sin_t = sin_; }
       const bool att_q = !(unfused & 2) && cfg_.head_dim == 128 && ly.wo.kind == MK_Q8;

@@ -877,7 +877,13 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
   // group L % ngroups, so the first workgroups on the CUs are the ones that stream the most of the cache and the short
   // ones fill in behind them (causal work grows with the tile index)
   const int L = blockIdx.y * gridDim.x + blockIdx.x;
-  const int bx = gridDim.x - 1 - L / gridDim.y, g = L % gridDim.y;
+  // with splits: the workgroups of one (group, share of its cache) on one XCD, whose L2 then reads that share once
+  int bx = gridDim.x - 1 - L / gridDim.y, g = L % gridDim.y, z = 0;
+  if (a.nsplit > 1) {
+    const int k = L >> 3, pair = k / gridDim.x * 8 + (L & 7);
+    if (pair >= a.nkv * a.nsplit) return;
+    bx = gridDim.x - 1 - k % gridDim.x; g = pair % a.nkv; z = pair / a.nkv;
+  }
   const int rep = a.nh / a.nkv, kvd = a.nkv * HD;
   const int ntiles = (a.ntok + 15) / 16, nunits = ntiles * rep;
   const int u = bx * kPfAttnWaves + wave;
@@ -890,7 +896,8 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
   // the workgroup streams up to its last live unit's last token
   const int ulast = min(bx * kPfAttnWaves + kPfAttnWaves - 1, nunits - 1);
   const int wg_last = a.p0 + min((ulast / rep) * 16 + 15, a.ntok - 1);
-  const int nkb = wg_last / kPfKB + 1;
+  // its cache blocks; with splits share z of them
+  const int nkb_all = wg_last / kPfKB + 1, kb0 = nkb_all * z / a.nsplit, nkb = nkb_all * (z + 1) / a.nsplit;
 
   // q^T fragments: lane holds q[t][32 s + 8 lg + 0..7] as hi / lo halves, pre-scaled by log2(e) / sqrt(hd) so the
   // scores come out in base-2 units for the hardware exp2 (v_exp_f32)
@@ -977,8 +984,8 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
     w[VS] = (lo_y & 0xffffu) | (hi_y << 16);
     w[3 * VS / 2] = (lo_y >> 16) | (hi_y & 0xffff0000u);
   };
-  load_block(0);
-  for (int kb = 0; kb < nkb; kb++) {
+  load_block(kb0 * kPfKB);
+  for (int kb = kb0; kb < nkb; kb++) {
     const int pb = kb * kPfKB;
     __syncthreads();   // the previous block's LDS reads are done
     store_piece(0, kr0, vr0);
@@ -1046,6 +1053,14 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
     }
   }
   if (!tok_ok) return;   // a token's four lanes (lr, l ^ 16, l ^ 32, l ^ 48) leave together
+  if (a.nsplit > 1) {   // unnormalised output and (max, sum) for k_pf_attn_merge (max -inf: no position in this share)
+    const size_t th = ((size_t)z * a.ntok + t) * a.nh + head;
+    if (lg == 0) *(float2 *)(a.part + (size_t)a.nsplit * a.ntok * a.nh * HD + 2 * th) = make_float2(m, l);
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+      *(float4 *)(a.part + th * HD + 16 * d + 4 * lg) = make_float4(o[d][0], o[d][1], o[d][2], o[d][3]);
+    return;
+  }
   const float inv = 1.f / l;
   if (HD == kQB && a.oh) {
     // quantise the head (one 128-column block; quant_rows as k_pf_quant: mx = max |v|, isx = mx > 0 ? 32767 / mx : 0,
@@ -1084,17 +1099,91 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
   for (int d = 0; d < DT; d++)
     *(float4 *)(out + 16 * d + 4 * lg) = make_float4(o[d][0] * inv, o[d][1] * inv, o[d][2] * inv, o[d][3] * inv);
 }
-hipError_t launch_pf_attn(const PfAttnArgs &a, hipStream_t st) {
+// The splits' outputs of one (token, head) per wave, lane l holding dims HD / 64 l ..: M = max m, L = sum l 2^(m - M),
+// out = sum o 2^(m - M) / L in split order, stored or (a.oh) quantised as k_pf_attn does.  Bound by reading the partials
+// once (150 tokens x 28 heads x 12 splits: 26 MB).
+template <int HD>
+__global__ __launch_bounds__(256) void k_pf_attn_merge(PfAttnArgs a) {
+  constexpr int D = HD / 64;
+  const int i = blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63, n = a.ntok * a.nh;
+  if (i >= n) return;
+  const int t = i / a.nh, head = i % a.nh;
+  const float *ml = a.part + (size_t)a.nsplit * n * HD;
+  float M = -INFINITY;
+  for (int z = 0; z < a.nsplit; z++) M = fmaxf(M, ml[2 * ((size_t)z * n + i)]);
+  float L = 0.f, v[D];
+#pragma unroll
+  for (int k = 0; k < D; k++) v[k] = 0.f;
+#pragma unroll 4
+  for (int z = 0; z < a.nsplit; z++) {
+    const float2 x = *(const float2 *)(ml + 2 * ((size_t)z * n + i));
+    const float f = x.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x.x - M);
+    L = __builtin_fmaf(x.y, f, L);
+    const float *o = a.part + ((size_t)z * n + i) * HD + D * lane;
+#pragma unroll
+    for (int k = 0; k < D; k++) v[k] = __builtin_fmaf(o[k], f, v[k]);
+  }
+  const float inv = 1.f / L;
+#pragma unroll
+  for (int k = 0; k < D; k++) v[k] *= inv;
+  if constexpr (HD == kQB) {
+    if (a.oh) {
+      const float mx = wave_max(fmaxf(fabsf(v[0]), fabsf(v[1])));
+      const float isx = mx > 0 ? kActMax / mx : 0.f;
+      if (lane == 0) {
+        const float bs = mx / kActMax;
+        a.ob[(size_t)t * a.ldb + head] = bs;
+        a.obt[(size_t)head * a.ldbt + t] = bs;
+      }
+      const int q0 = (int)__builtin_rintf(v[0] * isx), q1 = (int)__builtin_rintf(v[1] * isx), d = 2 * lane, p = d >> 4;
+      const size_t o = a.tiled ? (size_t)(t & ~15) * a.ldo + (size_t)head * 2048 + 16 * (t & 15) + 1024 * (p & 1) + 256 * (p >> 1) + (d & 15)
+                               : (size_t)t * a.ldo + head * HD + d;
+      *(uint16_t *)(a.oh + o) = (uint16_t)(((q0 >> 8) & 0xff) | ((q1 >> 8) & 0xff) << 8);
+      *(uint16_t *)(a.ol + o) = (uint16_t)(((q0 & 0xff) ^ 0x80) | ((q1 & 0xff) ^ 0x80) << 8);
+      return;
+    }
+  }
+  float *out = a.att + (size_t)t * a.lda + head * HD + D * lane;
+#pragma unroll
+  for (int k = 0; k < D; k++) out[k] = v[k];
+}
+
+// Splits of the cache per tile: few tokens behind a long context are a few dozen workgroups, each streaming the whole
+// cache at ~2.5 us per 64 positions (150 tokens, 28 heads in 4 groups at 12000: 36 workgroups, 430 us).  The split that is
+// expected to end first (here 6: 110 + 7 us): rounds of workgroups on the fullest XCD (the (group, share) pairs are dealt to the 8 XCDs, one
+// workgroup to a CU) times a share's blocks, then the merge (a launch and the partials); at least 4 blocks a share.
+static int pf_attn_splits(int gx, int nkv, int blocks, int cus, int most) {
+  const int per_xcd = std::max(1, cus / 8);
+  int best = 1;
+  double tbest = (double)((gx * nkv + cus - 1) / cus) * (blocks + 2.5) * 2.5;
+  for (int s = 2; s <= blocks / 4 && s <= most && s * gx * nkv <= 2 * cus; s++) {
+    const int on_xcd = (nkv * s + 7) / 8 * gx;
+    const double t = (double)((on_xcd + per_xcd - 1) / per_xcd) * ((blocks + s - 1) / s + 2.5) * 2.5 + 4 + 0.6 * s;
+    if (t < tbest) { tbest = t; best = s; }
+  }
+  return best;
+}
+hipError_t launch_pf_attn(const PfAttnArgs &a0, hipStream_t st) {
+  PfAttnArgs a = a0;
   if (a.ntok <= 0) return hipSuccess;
   if (a.nh % a.nkv || (a.hd != 64 && a.hd != 128) || a.lda % 4 || (a.cos_t && !a.sin_t)) return hipErrorInvalidValue;
   if (a.oh && (a.hd != kQB || !a.ol || !a.ob || !a.obt || a.ldo % 4 || a.ldbt < a.ntok)) return hipErrorInvalidValue;
   const int units = (a.ntok + 15) / 16 * (a.nh / a.nkv);
-  const dim3 grid((units + kPfAttnWaves - 1) / kPfAttnWaves, a.nkv);
+  dim3 grid((units + kPfAttnWaves - 1) / kPfAttnWaves, a.nkv);
+  const int blocks = (a.p0 + a.ntok - 1) / kPfKB + 1;
+  const int most = a.part ? (int)std::min<size_t>(64, a.part_floats / ((size_t)a.ntok * a.nh * (a.hd + 2))) : 1;   // splits that fit
+  a.nsplit = 1;
+  if (most > 1) a.nsplit = pf_attn_splits((int)grid.x, a.nkv, blocks, gemm_cus(), most);
+  if (const char *e = getenv("QPH_PF_SPLIT")) a.nsplit = std::max(1, std::min(most, atoi(e)));   // test hook
+  if (a.nsplit > 1) grid.y = (a.nkv * a.nsplit + 7) / 8 * 8;
   if (a.hd == 128) hipLaunchKernelGGL(k_pf_attn<128>, grid, dim3(kPfAttnWaves * 64), 0, st, a);
   else hipLaunchKernelGGL(k_pf_attn<64>, grid, dim3(kPfAttnWaves * 64), 0, st, a);
+  if (a.nsplit > 1) {
+    const dim3 mg((a.ntok * a.nh + 3) / 4);
+    if (a.hd == 128) hipLaunchKernelGGL(k_pf_attn_merge<128>, mg, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(k_pf_attn_merge<64>, mg, dim3(256), 0, st, a);
+  }
   return hipGetLastError();
 }
 
-// ------------------------------------------------------------------ SwiGLU of a token batch
-// g = silu(g) * u in place (silu_mul with exp256, kernels_x86.cpp:427-431, the decode epilogue's arithmetic)
 }  // namespace qph

@@ -292,6 +292,51 @@ def test_batched_prefill_q1(cfg, tile, n, synth, monkeypatch):
     gpu.close(); orc.close()
 
 
+@pytest.mark.parametrize("cfg,T,n", [("mini128", 900, 3), ("mini_r7h", 1500, 37), ("mini_r7", 800, 17), ("mini_q4m", 2000, 150),
+                                     ("mini_odd", 750, 16)])
+@pytest.mark.parametrize("split", ["", "2", "31"])
+def test_prefill_behind_a_long_context_splits(cfg, T, n, split, synth, monkeypatch):
+    """prompt attention whose cache is split over several workgroups per tile (few tokens behind a long context): logits
+    and the new cache rows against the unsplit kernel (QPH_PF_SPLIT=1) and the oracle's decode steps, with the launcher's
+    own split, two, and more than there are 64-position blocks at the shorter contexts (shares without a position); the
+    cache holds N(0, 1) rows and, past the context, NaN rows of a longer sequence"""
+    path = synth(cfg)
+    shape = qa.CONFIGS[cfg]
+    kvd = shape.kv_heads * shape.head_dim
+    rng = np.random.default_rng(T + n)
+    k = rng.standard_normal((shape.layers, T, kvd)).astype(np.float16)
+    v = rng.standard_normal((shape.layers, T, kvd)).astype(np.float16)
+    nan = np.full((shape.layers, n + 70, kvd), np.nan, np.float16)
+    snap = kv_snapshot(np.concatenate([k, nan], 1), np.concatenate([v, nan], 1))
+    toks = rng.integers(0, shape.vocab, n).astype(np.int32)
+    out = []
+    for s in ("1", split):
+        if s:
+            monkeypatch.setenv("QPH_PF_SPLIT", s)
+        else:
+            monkeypatch.delenv("QPH_PF_SPLIT")
+        print(f"{cfg}: {n} tokens behind {T}, split {s or 'auto'}", flush=True)
+        gpu = qa.HipLlama.load(path, max_ctx=T + n + 80)
+        gpu.restore(snap)
+        assert gpu.rewind(T)
+        out.append((gpu.prefill(toks, 1), split_snapshot(gpu.snapshot(), shape.layers, kvd)))
+        gpu.close()
+    assert np.isfinite(out[1][0]).all()
+    orc = O.Oracle(path, max_ctx=T + n + 80)
+    ko, vo = orc.kv_cache()
+    ko[:, :T] = k.view(np.uint16); vo[:, :T] = v.view(np.uint16)
+    orc.set_pos(T)
+    for t in toks:
+        lo = orc.step(int(t), 1)
+    for lg, _ in out:
+        err, ok = close(lg, lo)
+        assert ok, f"logits max|d| {err} against the oracle"
+    for a, b in zip(out[0][1][1:], out[1][1][1:]):
+        d = np.abs(a[:, T:].astype(np.float32) - b[:, T:].astype(np.float32))
+        assert d.max() <= 2e-3 * max(1.0, float(np.abs(a[:, T:].astype(np.float32)).max())), float(d.max())
+    orc.close()
+
+
 def kv_snapshot(k, v):
     """a snapshot in the reference layout (model_llama.cpp:55-63) from per-layer fp16 K / V rows [L][pos][kvd]"""
     pos = k.shape[1]
