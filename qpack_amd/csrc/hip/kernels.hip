@@ -438,6 +438,7 @@ __global__ __launch_bounds__(1024) void k_matvec(MvArgs a) {
   }
 }
 
+MvConfig g_mv_config;
 // rows per unit: SwiGLU units are one gate/up row pair; large matrices stream 2 rows per unit (the activation LDS reads
 // serve both), small ones 1 row so every wave gets an equal share
 static int mv_ns(const MvArgs &a, int epi, int waves) {
@@ -458,6 +459,30 @@ void mv_plan(MvArgs &a, int epi) {
 
 // Launch shape: every CU gets one workgroup of `w` waves and every wave the same number of units, where possible:
 // units per CU upc = ceil(U / cus); w = the largest divisor of upc in [4, 16] (16 when there is none).
+static void mv_shape(int units, int cols, int epi, int cus, int &w, int &grid) {
+  const int upc = (units + cus - 1) / cus;
+  // at most 8 waves per workgroup for gate / up and the head, 16 for the rest (same-box sweep, C3 greedy: 16
+  // everywhere 513.9 tok/s, 8 for gate / up and head 521.7, 12 for all 521.1, 6 or 4 for gate / up and head ~467)
+  const int WM = epi == EPI_SWIGLU || epi == EPI_ARGMAX ? 8 : 16;
+  w = upc <= WM ? upc : WM;
+  if (upc > WM) for (int c = WM; c >= 4; c--) if (upc % c == 0) { w = c; break; }
+  int u = (upc + w - 1) / w;                                        // units per wave
+  if (cols / kQB > 2 * w * 8) { w = 16; u = (upc + 15) / 16; }     // the prologue covers 2 x (threads / 8) blocks
+  grid = (units + w * u - 1) / (w * u);
+  // units are dealt round-robin over all the launch's waves, so a grid short of the CU count (units per CU with no
+  // divisor in 4..16) only leaves CUs idle: one workgroup per CU then
+  if (grid < cus && units >= cus) grid = cus;
+}
+MvDeal mv_deal(const DMat &m, int epi) {
+  MvArgs a{}; a.m[0] = m; a.nseg = 1;
+  MvDeal d{};
+  d.ns = mv_ns(a, epi, g_mv_config.cus * 16);
+  d.units = epi == EPI_SWIGLU ? m.rows : (m.rows + d.ns - 1) / d.ns;
+  int w, grid;
+  mv_shape(d.units, m.cols, epi, g_mv_config.cus, w, grid);
+  d.waves = w * grid;
+  return d;
+}
 template <int PRO, int EPI, int NS, int KIND>
 static hipError_t launch_mv_t(MvArgs a, int grid_cap, hipStream_t st) {
   if (EPI != EPI_SWIGLU) {
@@ -466,19 +491,9 @@ static hipError_t launch_mv_t(MvArgs a, int grid_cap, hipStream_t st) {
     a.seg_tile0[a.nseg] = t;
   }
   const int units = a.seg_tile0[a.nseg], cus = g_mv_config.cus;
-  const int upc = (units + cus - 1) / cus;
-  // at most 8 waves per workgroup for gate / up and the head, 16 for the rest (same-box sweep, C3 greedy: 16
-  // everywhere 513.9 tok/s, 8 for gate / up and head 521.7, 12 for all 521.1, 6 or 4 for gate / up and head ~467)
-  constexpr int WM = EPI == EPI_SWIGLU || EPI == EPI_ARGMAX ? 8 : 16;
-  int w = upc <= WM ? upc : WM;
-  if (upc > WM) for (int c = WM; c >= 4; c--) if (upc % c == 0) { w = c; break; }
-  int u = (upc + w - 1) / w;                                        // units per wave
   const int cols = a.m[0].cols;
-  if (cols / kQB > 2 * w * 8) { w = 16; u = (upc + 15) / 16; }     // the prologue covers 2 x (threads / 8) blocks
-  int grid = (units + w * u - 1) / (w * u);
-  // units are dealt round-robin over all the launch's waves, so a grid short of the CU count (units per CU with no
-  // divisor in 4..16) only leaves CUs idle: one workgroup per CU then
-  if (grid < cus && units >= cus) grid = cus;
+  int w, grid;
+  mv_shape(units, cols, EPI, cus, w, grid);
   if (grid > grid_cap) return hipErrorInvalidValue;
   // a wave may own one unit more than u when the grid rounds: size the per-wave LDS for ceil(units / waves)
   const int waves = grid * w;
@@ -527,7 +542,6 @@ static hipError_t launch_mv_k(int pro, int epi, const MvArgs &a, int ns, int gri
   if (pro == PRO_NORM_SUM && epi == EPI_SWIGLU) return launch_mv_t<PRO_NORM_SUM, EPI_SWIGLU, 2, KIND>(a, grid_cap, st);
   return hipErrorInvalidValue;
 }
-MvConfig g_mv_config;
 // grid_cap: the most workgroups one launch may use (EPI_ARGMAX writes one (max, index) partial per workgroup).
 // Segments of q8 and q4 (q4m: q4 wq / wk with a q8 wv) go out as one MK_MIX launch of the stored-output kernels, where
 // each wave streams one kind; other mixes (q1) as one launch per kind.
@@ -740,7 +754,7 @@ __device__ __forceinline__ void mf_dma_v(const uint16_t *vc, int kvd, int g, int
 struct AttnNoMid { __device__ void operator()() const {} };
 template <int HD, int REP, bool ONE = false, typename Mid = AttnNoMid, typename Epi = AttnNoEpi>
 __device__ void attn_split(const AttnArgs &a, int g, int s, int S, int ys, float *lout = nullptr, const Mid &mid = Mid(),
-                           const Epi &epi = Epi()) {
+                           const Epi &epi = Epi(), int tok = 0) {
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   typedef float f4 __attribute__((ext_vector_type(4)));
   typedef short s4 __attribute__((ext_vector_type(4)));
@@ -779,7 +793,7 @@ __device__ void attn_split(const AttnArgs &a, int g, int s, int S, int ys, float
       qh[k] = __builtin_bit_cast(h8, h); ql[k] = __builtin_bit_cast(h8, lo);
     }
   }
-  const int pos = ctl_pos_wait(pos_s), T = pos + 1;
+  const int pos = ctl_pos_wait(pos_s) + tok, T = pos + 1;
   const int t0 = (int)((int64_t)s * T / S), t1 = (int)((int64_t)(s + 1) * T / S);
   // wave w takes blocks w, w + NW, ... of the split's 32-position blocks (waves without a block idle)
   const int nblk = (t1 - t0 + kAttnMfBlk - 1) / kAttnMfBlk, nact = min(nblk, NW);
@@ -903,7 +917,7 @@ __device__ void attn_split(const AttnArgs &a, int g, int s, int S, int ys, float
 // at once, together with wave j's loads of head j's (m, l) pairs (one split per lane); wave j then forms head j's
 // factors e^(m_c - M) and 1 / L, and the column sums go through LDS.
 template <int HD, int REP, int NW>
-__device__ void attn_merge_all(const AttnArgs &a, int g, int S) {
+__device__ void attn_merge_all(const AttnArgs &a, int g, int S, int ys) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   auto cload = [](const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
   constexpr int NC = REP * HD / 4;                            // output columns of 4 dims
@@ -911,12 +925,12 @@ __device__ void attn_merge_all(const AttnArgs &a, int g, int S) {
   constexpr int K = (kAttnParMerge - 1 + P - 1) / P;          // loads per thread
   __shared__ float fw[REP][kAttnParMerge], linv[REP];
   __shared__ float4 opart[NW * 64];
-  const float *ml = a.part + (size_t)a.nh * gridDim.y * HD + 2 * (size_t)g * REP * gridDim.y;
+  const float *ml = a.part + (size_t)a.nh * ys * HD + 2 * (size_t)g * REP * ys;
   const int e = threadIdx.x % NC, part = threadIdx.x / NC;
   const int j = e / (HD / 4), i4 = e % (HD / 4);
   f32x4 v[K];
   if (part < P) {
-    const float4 *ph = (const float4 *)(a.part + ((size_t)(g * REP + j) * gridDim.y) * HD) + i4;
+    const float4 *ph = (const float4 *)(a.part + ((size_t)(g * REP + j) * ys) * HD) + i4;
 #pragma unroll
     for (int k = 0; k < K; k++) {   // clamped in range; unused ones are not summed
       const int c = part + k * P < S ? part + k * P : 0;
@@ -925,7 +939,7 @@ __device__ void attn_merge_all(const AttnArgs &a, int g, int S) {
   }
   if (wave < REP) {
     const bool on = lane < S;
-    const float *mp = ml + 2 * ((size_t)wave * gridDim.y + lane);
+    const float *mp = ml + 2 * ((size_t)wave * ys + lane);
     const float2 mv = on ? make_float2(cload(mp), cload(mp + 1)) : make_float2(-INFINITY, 0.f);
     const float M = wave_max(mv.x);
     const float f = on && mv.x != -INFINITY ? expf(mv.x - M) : 0.f;
@@ -1016,10 +1030,16 @@ __device__ void attn_merge_heads(const AttnArgs &a, int g, int S, int r, int MG,
   }
 }
 
+// token z of a batch (AttnArgs::ntok): its queries, outputs and partials, its position ctl->pos + z
+template <int HD>
+__device__ __forceinline__ void attn_token(AttnArgs &a, int z) {
+  a.q16 += (size_t)z * 2 * a.nh * HD; a.att += (size_t)z * a.nh * HD; a.part += (size_t)z * a.nh * a.max_chunks * (HD + 2);
+}
 template <int HD, int REP>
 __global__ __launch_bounds__(kAttnMfWaves * 64) void k_attention(AttnArgs a) {
   constexpr int NW = kAttnMfWaves;
-  const int pos = a.ctl->pos, T = pos + 1, g = blockIdx.x, s = blockIdx.y;
+  attn_token<HD>(a, blockIdx.z);
+  const int pos = a.ctl->pos + blockIdx.z, T = pos + 1, g = blockIdx.x, s = blockIdx.y;
   // one workgroup per kv group while the group's K and V are at most 64 KiB (a CU streams ~55 GB/s: 128 positions at
   // head dim 128, 256 at 64); beyond that up to 64 splits of >= 64 positions
   const int smax = a.single_max > 0 ? a.single_max : kAttnMfBlk * NW * 64 / HD, sp = a.split_pos > 0 ? a.split_pos : 64;
@@ -1027,7 +1047,7 @@ __global__ __launch_bounds__(kAttnMfWaves * 64) void k_attention(AttnArgs a) {
   if (s >= S) return;
   uint64_t st0 = 0, st1 = 0, st2 = 0;   // measurement (a.stamps): start, partials stored, rank known
   if (a.stamps) st0 = __builtin_amdgcn_s_memrealtime();
-  attn_split<HD, REP>(a, g, s, S, gridDim.y);
+  attn_split<HD, REP>(a, g, s, S, gridDim.y, nullptr, AttnNoMid(), AttnNoEpi(), blockIdx.z);
   if (S == 1 || (a.merge_sep && S >= a.merge_sep)) return;   // merge_sep: k_attn_merge merges (the next launch)
   // this thread's coherent stores have completed before the workgroup's counter bump
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1069,7 +1089,7 @@ __global__ __launch_bounds__(kAttnMfWaves * 64) void k_attention(AttnArgs a) {
   // The partials were written through to memory by other workgroups before their counter bumps; they are read with
   // coherent loads (no acquire fence: that is an L2 invalidate, far slower).
   if (S < kAttnParMerge) {
-    attn_merge_all<HD, REP, NW>(a, g, S);
+    attn_merge_all<HD, REP, NW>(a, g, S, gridDim.y);
     stamp(1);
     return;
   }
@@ -1095,6 +1115,21 @@ __global__ __launch_bounds__(kAttnMfWaves * 64) void k_attn_merge(AttnArgs a) {
   attn_merge_heads<HD, REP, kAttnMfWaves>(a, blockIdx.x, S, blockIdx.y, REP, false, a.max_chunks);
 }
 
+// The same for a batch of tokens (grid (group, head of the group, token)): every split count is merged here, with the
+// arithmetic a decode step at that position uses - one workgroup for all heads below kAttnParMerge splits, else one a head
+template <int HD, int REP>
+__global__ __launch_bounds__(kAttnMfWaves * 64) void k_attn_merge_batch(AttnArgs a) {
+  attn_token<HD>(a, blockIdx.z);
+  const int T = a.ctl->pos + blockIdx.z + 1;
+  const int smax = a.single_max > 0 ? a.single_max : kAttnMfBlk * kAttnMfWaves * 64 / HD, sp = a.split_pos > 0 ? a.split_pos : 64;
+  const int S = T <= smax ? 1 : min(a.max_chunks, (T + sp - 1) / sp);
+  if (S == 1) return;
+  if (S >= kAttnParMerge || (a.heads_min > 0 && T >= a.heads_min))
+    attn_merge_heads<HD, REP, kAttnMfWaves>(a, blockIdx.x, S, blockIdx.y, REP, false, a.max_chunks);
+  else if (blockIdx.y == 0)
+    attn_merge_all<HD, REP, kAttnMfWaves>(a, blockIdx.x, S, a.max_chunks);
+}
+
 int attn_long_merge_min(int hd, int single_max, int split_pos, int max_chunks, int min_splits) {
   const int smax = single_max > 0 ? single_max : kAttnMfBlk * kAttnMfWaves * 64 / hd, sp = split_pos > 0 ? split_pos : 64;
   if (min_splits < 2 || max_chunks < min_splits) return 0;
@@ -1103,12 +1138,16 @@ int attn_long_merge_min(int hd, int single_max, int split_pos, int max_chunks, i
 
 hipError_t launch_attention(const AttnArgs &a, hipStream_t st) {
   if (a.nh % a.nkv || a.nh / a.nkv > 8 || a.max_chunks < 1 || a.max_chunks > kAttnMaxSplits) return hipErrorInvalidValue;
-  const dim3 grid(a.nkv, a.max_chunks);
+  const int nt = std::max(1, a.ntok);
+  if (nt > 1 && (a.max_chunks > 1) != (a.merge_sep == 2)) return hipErrorInvalidValue;   // a batch never merges in-kernel
+  const dim3 grid(a.nkv, a.max_chunks, nt);
   const int rep = a.nh / a.nkv;
 #define QPH_ATT(HD, R)                                                                                              \
   if (a.hd == HD && rep == R) {                                                                                     \
     hipLaunchKernelGGL((k_attention<HD, R>), grid, dim3(kAttnMfWaves * 64), 0, st, a);                              \
-    if (a.merge_sep) hipLaunchKernelGGL((k_attn_merge<HD, R>), dim3(a.nkv, R), dim3(kAttnMfWaves * 64), 0, st, a);   \
+    if (nt > 1 && a.merge_sep)                                                                                      \
+      hipLaunchKernelGGL((k_attn_merge_batch<HD, R>), dim3(a.nkv, R, nt), dim3(kAttnMfWaves * 64), 0, st, a);       \
+    else if (a.merge_sep) hipLaunchKernelGGL((k_attn_merge<HD, R>), dim3(a.nkv, R), dim3(kAttnMfWaves * 64), 0, st, a);   \
     return hipGetLastError();                                                                                       \
   }
   QPH_ATT(64, 1) QPH_ATT(64, 2) QPH_ATT(64, 3) QPH_ATT(64, 4) QPH_ATT(64, 5) QPH_ATT(64, 6) QPH_ATT(64, 7) QPH_ATT(64, 8)

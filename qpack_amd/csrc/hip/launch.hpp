@@ -83,6 +83,10 @@ constexpr int kMvMaxWaves = 16;
 constexpr int kMvSlots = 2;
 int mv_tile_rows(int epi);
 size_t mv_lds_bytes(int cols, int waves, int per_wave);
+// how launch_matvec deals a single q8 matrix's (or gate / up pair's) rows to waves: units of ns rows (SwiGLU: one row of
+// each matrix), unit u to wave u % waves - which decides how many lanes chain a row's blocks (MvArgs::split_chain)
+struct MvDeal { int ns, units, waves; };
+MvDeal mv_deal(const DMat &m, int epi);
 // fills seg_tile0 from the segment row counts
 void mv_plan(MvArgs &a, int epi);
 // grid_cap: the most workgroups (EPI_ARGMAX writes one (max, index) partial per workgroup launched)
@@ -122,6 +126,10 @@ struct AttnArgs {
                                // the context is known (0: all); the others load theirs, if they have one, once it is
   int merge_sep;               // > 1: contexts of at least this many splits only store their partials and a second
                                // launch (k_attn_merge, one workgroup per head) merges them
+  // ntok > 1: a batch of tokens at positions ctl->pos .. + ntok - 1 (their cache rows all written): q16 [ntok][2 nh hd],
+  // att [ntok][nh * hd], part one share of nh * max_chunks * (hd + 2) floats per token; merge_sep 2 unless max_chunks is 1.
+  // heads_min: the context from which decode steps merge in a launch of their own (0: never)
+  int ntok, heads_min;
   uint64_t *stamps;            // measurement only (optional): per workgroup of k_attention 5 words - realtime at start,
                                // partials stored, merge rank known, end, and 1 if it merged
 };
@@ -219,6 +227,11 @@ struct GemmArgs {
   // segment fields replacing w / scale / wsum / st / bias / y / ldy / rows; each starts on a fresh row tile
   int nseg;
   GemmSeg seg[kGemmMaxSeg];
+  // few-token kernel only: another fp32 order of the block sums than rows_q8's single chain, as the decode step's kernels
+  // have it - deal.waves > 0: MvArgs::split_chain of a matvec dealt like that; group_blocks > 0: a chain of its own per
+  // group_blocks blocks, scaled, the groups then summed in order (k_attn_wo)
+  MvDeal deal;
+  int group_blocks;
   int tile0;   // first row tile of this launch (a launch split over the two q8 kernels; set by launch_gemm)
   int dbg;   // measurement switches of the 32 x 32 q8 kernel (QPH_G2_DBG; results are wrong when set): 1 no compute,
              // 2 no loads after the first block, 4 no barriers
@@ -251,6 +264,7 @@ struct PfRopeArgs {
   uint16_t *kc, *vc;
   int p0, nh, nkv, hd;
   int skip_q;   // q is rotated by the attention kernel instead
+  uint16_t *q16;   // optional (with q rotated here): q as fp16 hi [nh * hd] then lo halves per token, as MvArgs::q16
 };
 hipError_t launch_pf_rope(const PfRopeArgs &a, int B, hipStream_t st);
 // causal attention of the batch's (rotated) queries over cache positions [0, p0 + t] -> att [t][lda]

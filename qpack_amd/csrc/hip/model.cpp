@@ -211,6 +211,11 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
     pf_xbt2_ = (float *)dalloc(4ull * pf_ldbt_ * (pf_ldq_ / 128 + 1));
     if (half_mats) pf_fp_ = (uint16_t *)dalloc(4 * B16 * wide);
     pf_tok_ = (int *)dalloc(4 * B);
+    // batched prefill_all: q8 throughout, the scratch (the gate / up output's buffer: attention partials, logits) fits, and
+    // the fused attention adds its parts itself
+    vf_ok_ = !half_mats && head_.kind == MK_Q8 && (awo_max_ <= 0 || awo_rows_ || awo_sum_) && B >= (size_t)kVerify &&
+             B * ff >= (size_t)kVerify * std::max<size_t>(V, (size_t)nh * max_chunks_ * (hd + 2));
+    if (vf_ok_) vf_q16_ = (uint16_t *)dalloc(4ull * kVerify * qd_);
   }
   // RoPE tables in the reference's precision: inv_i = 1 / theta^(2i/hd) and angle pos * inv_i in double, cos / sin
   // rounded to float (model_llama.cpp:39, :173-175)
@@ -252,6 +257,8 @@ HipLlama::~HipLlama() {
   if (hctl_) (void)hipHostFree(hctl_);
   if (hout_) (void)hipHostFree(hout_);
   if (htok_) (void)hipHostFree(htok_);
+  if (vf_host_) (void)hipHostFree(vf_host_);
+  for (hipEvent_t e : vf_ev_) if (e) (void)hipEventDestroy(e);
   if (htopk_) (void)hipHostFree(htopk_);
   if (hstatus_) (void)hipHostFree(hstatus_);
   if (st_) (void)hipStreamDestroy(st_);
@@ -676,9 +683,97 @@ int HipLlama::greedy_run(int tok, int n, int *out) {
   return n;
 }
 
+// Model::prefill_all: every token's logits equal its decode step's bit for bit (the reference's ExactBatches contract).
+// q8 models in the default order: batches of up to kVerify tokens through products that read the weights once and sum in
+// the decode kernels' orders; a batch stays on one side of the fused attention's limit, whose order differs.
 void HipLlama::prefill_all(const int *toks, int n, float *logits) {
   if (pos_ + n > ctx_) throw std::runtime_error("context window full (" + std::to_string(ctx_) + " tokens)");
-  for (int i = 0; i < n; i++) step(toks[i], 1, logits + (size_t)i * cfg_.vocab);
+  const bool batched = vf_ok_ && !order_ && !getenv("QPH_VERIFY_STEPS");   // test hook: decode steps
+  for (int i = 0; i < n;) {
+    int m = 0;   // tokens of this batch: valid ids, one regime
+    const bool fused = pos_ + 1 <= awo_max_;
+    while (batched && m < kVerify && i + m < n && toks[i + m] >= 0 && toks[i + m] < cfg_.vocab &&
+           (pos_ + m + 1 <= awo_max_) == fused) m++;
+    if (m > 1) { verify_batch(toks + i, m, fused, logits + (size_t)i * cfg_.vocab); i += m; }
+    else { step(toks[i], 1, logits + (size_t)i * cfg_.vocab); i++; }
+  }
+}
+
+void HipLlama::verify_batch(const int *toks, int n, bool fused, float *logits) {
+  const int d = cfg_.hidden, ff = cfg_.ffn, V = cfg_.vocab;
+  if (!vf_host_) {
+    QPH_CK(hipHostMalloc((void **)&vf_host_, 4ull * V, hipHostMallocDefault));
+    for (hipEvent_t &e : vf_ev_) QPH_CK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  auto quant = [&](int pro, const float *x, int ldx, const float *w, int cols) {
+    PfQuantArgs a{}; a.x = x; a.ldx = ldx; a.norm_w = w; a.eps = cfg_.rms_eps; a.cols = cols;
+    a.th = pf_th_; a.tl = pf_tl_; a.ldq = pf_ldq_; a.xb = pf_xb_; a.ldb = pf_ldb_;
+    QPH_CK(launch_pf_quant(pro, a, n, st_));
+  };
+  auto product = [&](const DMat &m, float *y, int ldy) {
+    GemmArgs a{}; a.kind = MK_Q8; a.w = (const int8_t *)m.q; a.scale = (const float *)m.s; a.rows = m.rows; a.cols = m.cols;
+    a.th = pf_th_; a.tl = pf_tl_; a.xb = pf_xb_; a.ntok = n; a.ldq = pf_ldq_; a.ldb = pf_ldb_; a.y = y; a.ldy = ldy;
+    return a;
+  };
+  const int p0 = pos_;
+  write_ctl(toks[0], p0);
+  QPH_CK(hipMemcpyAsync(pf_tok_, toks, 4ull * n, hipMemcpyHostToDevice, st_));
+  QPH_CK(launch_pf_embed(embed_, pf_tok_, n, pf_x_, d, st_));
+  for (int l = 0; l < cfg_.layers; l++) {
+    const Layer &ly = layers_[l];
+    uint16_t *kc = kc_ + (size_t)l * ctx_ * kvd_, *vc = vc_ + (size_t)l * ctx_ * kvd_;
+    quant(PRO_NORM, pf_x_, d, ly.an, d);
+    {
+      const DMat *m[3] = {&ly.wq, &ly.wk, &ly.wv};
+      float *y[3] = {pf_q_, pf_k_, pf_v_};
+      const int ld[3] = {qd_, kvd_, kvd_};
+      const float *bias[3] = {ly.bq, ly.bk, ly.bv};
+      GemmArgs a = product(ly.wq, pf_q_, qd_);
+      a.nseg = 3;
+      for (int s = 0; s < 3; s++) a.seg[s] = GemmSeg{(const int8_t *)m[s]->q, (const float *)m[s]->s, m[s]->rs, nullptr, bias[s], y[s], m[s]->rows, ld[s]};
+      QPH_CK(launch_gemm(a, st_));
+    }
+    PfRopeArgs r{}; r.q = pf_q_; r.ldq = qd_; r.k = pf_k_; r.v = pf_v_; r.ldk = kvd_; r.cos_t = cos_; r.sin_t = sin_;
+    r.kc = kc; r.vc = vc; r.p0 = p0; r.nh = cfg_.heads; r.nkv = cfg_.kv_heads; r.hd = cfg_.head_dim; r.q16 = vf_q16_;
+    QPH_CK(launch_pf_rope(r, n, st_));
+    AttnArgs at{}; at.q16 = vf_q16_; at.ctx = ctx_; at.kc = kc; at.vc = vc; at.ctl = ctl_; at.part = pf_g_; at.att = pf_att_;
+    at.nh = cfg_.heads; at.nkv = cfg_.kv_heads; at.hd = cfg_.head_dim; at.ntok = n; at.heads_min = lm_min_;
+    // the fused kernels run one split whatever the context
+    at.max_chunks = fused ? 1 : max_chunks_; at.single_max = fused ? ctx_ : attn_single_; at.split_pos = attn_split_pos_;
+    at.merge_sep = at.max_chunks > 1 ? 2 : 0;
+    QPH_CK(launch_attention(at, st_));
+    quant(PRO_QUANT, pf_att_, qd_, nullptr, qd_);
+    GemmArgs wo = product(ly.wo, pf_x_, d);
+    wo.resid = 1;
+    if (fused && !awo_rows_) wo.group_blocks = qd_ / cfg_.kv_heads / 128;   // k_attn_wo: a chain per kv group
+    QPH_CK(launch_gemm(wo, st_));
+    quant(PRO_NORM, pf_x_, d, ly.fn, d);
+    GemmArgs gu = product(ly.wg, pf_g_, ff);
+    gu.w2 = (const int8_t *)ly.wu.q; gu.scale2 = (const float *)ly.wu.s; gu.wsum2 = ly.wu.rs;
+    if (split_chain_) gu.deal = mv_deal(ly.wg, EPI_SWIGLU);
+    QPH_CK(launch_gemm(gu, st_));
+    quant(PRO_QUANT, pf_g_, ff, nullptr, ff);
+    GemmArgs dn = product(ly.wd, pf_x_, d);
+    dn.resid = 1;
+    if (split_chain_) dn.deal = mv_deal(ly.wd, EPI_RESID);
+    QPH_CK(launch_gemm(dn, st_));
+  }
+  quant(PRO_NORM, pf_x_, d, fnorm_, d);
+  QPH_CK(launch_gemm(product(head_, pf_g_, V), st_));
+  pos_ += n;
+  // the rows to the host through two pinned buffers: a row is copied out while the next one arrives
+  float *hb[2] = {hout_, vf_host_};
+  auto fetch = [&](int i) {
+    QPH_CK(hipMemcpyAsync(hb[i & 1], pf_g_ + (size_t)i * V, 4ull * V, hipMemcpyDeviceToHost, st_));
+    QPH_CK(hipEventRecord(vf_ev_[i & 1], st_));
+  };
+  fetch(0);
+  for (int i = 0; i < n; i++) {
+    if (i + 1 < n) fetch(i + 1);
+    QPH_CK(hipEventSynchronize(vf_ev_[i & 1]));
+    if (i == 0) check_status();
+    memcpy(logits + (size_t)i * V, hb[i & 1], 4ull * V);
+  }
 }
 
 void HipLlama::set_pos(int pos) {

@@ -153,6 +153,13 @@ class HipLlama {
   uint16_t *pf_fp_ = nullptr;   // fp16 planes (PfQuantArgs::fp), for models with q4 or q1 layers
   int *pf_tok_ = nullptr;
   void prefill_batched(const int *toks, int n);
+  // prefill_all in batches of up to kVerify tokens whose every logit equals its decode step's bit for bit (q8 models)
+  static constexpr int kVerify = 16;
+  bool vf_ok_ = false;
+  uint16_t *vf_q16_ = nullptr;   // [kVerify][2 qd_]
+  float *vf_host_ = nullptr;     // pinned: the second row buffer of the logits' way to the host
+  hipEvent_t vf_ev_[2] = {};
+  void verify_batch(const int *toks, int n, bool fused, float *logits);
 
   void *dalloc(size_t bytes);
   DMat upload(const qph_tensor &t);

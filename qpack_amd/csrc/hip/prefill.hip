@@ -822,6 +822,16 @@ __global__ __launch_bounds__(256) void k_pf_rope(PfRopeArgs a) {
     float *qh = q + h * a.hd; const float x0 = qh[i], x1 = qh[i + half];
     qh[i] = __builtin_fmaf(x0, cs[i], -(x1 * sn[i]));
     qh[i + half] = __builtin_fmaf(x1, cs[i], x0 * sn[i]);
+    if (a.q16) {
+      uint16_t *hp = a.q16 + (size_t)t * 2 * a.nh * a.hd + h * a.hd, *lp = hp + a.nh * a.hd;
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        const float y = qh[i + k * half];
+        const _Float16 hv = (_Float16)y;
+        hp[i + k * half] = __builtin_bit_cast(uint16_t, hv);
+        lp[i + k * half] = __builtin_bit_cast(uint16_t, (_Float16)(y - (float)hv));
+      }
+    }
   }
   const float *k = a.k + (size_t)t * a.ldk, *v = a.v + (size_t)t * a.ldk;
   uint16_t *kr = a.kc + (size_t)pos * kvd, *vr = a.vc + (size_t)pos * kvd;

@@ -41,7 +41,10 @@ __device__ __forceinline__ void lds_barrier() {
 // per wave and round bound it (without any loads 40 tokens take 20 of 37 us).
 // Depth: 2 rounds of each; 4 of the weights, or of both, were slower (4096 x 14336, 16 tokens 20.2 / 21.0 / 21.9 us).
 constexpr int kSkWaves = 8, kSkDepth = 2;
-template <int RT, int NTT, int DA, int DB>
+// ORD: the fp32 order of a row's block sums.  0: one chain; 1: the decode matvec's split chain - shares of the blocks
+// chained each from zero, then summed pairwise; the share sums wait in LDS; 2: k_attn_wo's - a chain per kv group times the
+// row scale, the groups summed in order.  1 and 2 give a token's row the bits its decode step gives it.
+template <int RT, int NTT, int DA, int DB, int ORD>
 __global__ __launch_bounds__(kSkWaves * 64) void k_skinny_q8(GemmArgs a, int nrt, int ntk) {
   constexpr int RW = 16 * RT, NT = 16 * NTT, P = RW + 4;   // rows, tokens, floats between two tokens' rows in LDS
   extern __shared__ __align__(16) float sums[];            // [2 rounds][8 blocks][NT][P]
@@ -137,7 +140,21 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_skinny_q8(GemmArgs a, int nrt
   Tile tl = tile_of(rt0);
   int ctile = 0, cround = 0;
   float4 sc4, ex4;
+  float *shares = sums + 2 * kSkWaves * NT * P + tid;   // ORD 1: [4 rows][8 shares][chain threads]
+  constexpr int CT = NT * RW / 4;
+  int share_len[4], left[4], nshare[4];                      // ORD 1: blocks per share, left in it, shares stored
+  float4 ysum = make_float4(0.f, 0.f, 0.f, 0.f);             // ORD 2
+  int gleft = a.group_blocks;
   auto load_c = [&]() {
+    if constexpr (ORD == 1) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int r = tl.r0 + (paired ? 4 * (cq & 3) : 4 * cq) + i, gw = (paired ? r : r / a.deal.ns) % a.deal.waves;
+        const int n = (a.deal.units - gw + a.deal.waves - 1) / a.deal.waves * a.deal.ns;   // rows of the wave that has this one
+        const int lanes = n <= 8 ? 8 : n <= 16 ? 4 : n <= 32 ? 2 : 1;
+        share_len[i] = left[i] = (nb + 4 * lanes - 1) / (4 * lanes) * 4; nshare[i] = 0;
+      }
+    }
     const int row = min(tl.r0 + (paired ? 4 * (cq & 3) : 4 * cq), tl.rows - 1), n4 = min(3, tl.rows - 1 - row);
     const float *sc = (paired && cq >= 4 ? tl.scale2 : tl.scale) + row;
     sc4 = make_float4(sc[0], sc[min(1, n4)], sc[min(2, n4)], sc[n4]);
@@ -193,26 +210,55 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_skinny_q8(GemmArgs a, int nrt
       const float *sp = sb + ct * P + 4 * cq;
       const float4 w0 = bs[par][0], w1 = bs[par][1];
       const float wv[kSkWaves] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-      auto fold = [&](float w, const float4 &s) {
-        acc.x = __builtin_fmaf(w, s.x, acc.x); acc.y = __builtin_fmaf(w, s.y, acc.y);
-        acc.z = __builtin_fmaf(w, s.z, acc.z); acc.w = __builtin_fmaf(w, s.w, acc.w);
+      auto fold = [&](int j, const float4 &s) {
+        acc.x = __builtin_fmaf(wv[j], s.x, acc.x); acc.y = __builtin_fmaf(wv[j], s.y, acc.y);
+        acc.z = __builtin_fmaf(wv[j], s.z, acc.z); acc.w = __builtin_fmaf(wv[j], s.w, acc.w);
+        if constexpr (ORD == 1) {
+          if ((j & 3) == 3 || b0 + j == nb - 1) {   // shares are whole multiples of four blocks, the last may end early
+            float *ap[4] = {&acc.x, &acc.y, &acc.z, &acc.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              left[i] -= 4;
+              if (left[i] == 0 || b0 + j == nb - 1) { shares[(8 * i + nshare[i]++) * CT] = *ap[i]; *ap[i] = 0.f; left[i] = share_len[i]; }
+            }
+          }
+        }
+        if constexpr (ORD == 2) {
+          if (--gleft == 0) {
+            float4 p = make_float4(acc.x * sc4.x, acc.y * sc4.y, acc.z * sc4.z, acc.w * sc4.w);
+            asm volatile("" : "+v"(p.x), "+v"(p.y), "+v"(p.z), "+v"(p.w));   // rounded parts, then added
+            ysum.x += p.x; ysum.y += p.y; ysum.z += p.z; ysum.w += p.w;
+            acc = make_float4(0.f, 0.f, 0.f, 0.f); gleft = a.group_blocks;
+          }
+        }
       };
       if (b0 + kSkWaves <= nb) {
         float4 s[kSkWaves];
 #pragma unroll
         for (int j = 0; j < kSkWaves; j++) s[j] = *(const float4 *)(sp + j * (NT * P));
 #pragma unroll
-        for (int j = 0; j < kSkWaves; j++) fold(wv[j], s[j]);
+        for (int j = 0; j < kSkWaves; j++) fold(j, s[j]);
       } else {
 #pragma unroll
         for (int j = 0; j < kSkWaves - 1; j++)
-          if (b0 + j < nb) fold(wv[j], *(const float4 *)(sp + j * (NT * P)));
+          if (b0 + j < nb) fold(j, *(const float4 *)(sp + j * (NT * P)));
       }
     }
     if (++cround < rounds) return;
     cround = 0;
     if (chain) {
+      if constexpr (ORD == 1) {   // ((c0 + c1) + (c2 + c3)) + ((c4 + c5) + (c6 + c7)), absent shares zero
+        float *ap[4] = {&acc.x, &acc.y, &acc.z, &acc.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float c[8];
+#pragma unroll
+          for (int k = 0; k < 8; k++) c[k] = k < nshare[i] ? shares[(8 * i + k) * CT] : 0.f;
+          *ap[i] = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+        }
+      }
       float v[4] = {acc.x * sc4.x, acc.y * sc4.y, acc.z * sc4.z, acc.w * sc4.w};
+      if constexpr (ORD == 2) { v[0] = ysum.x; v[1] = ysum.y; v[2] = ysum.z; v[3] = ysum.w; ysum = make_float4(0.f, 0.f, 0.f, 0.f); }
       float *yt = tl.y + (size_t)ctok * tl.ldy;
       if (paired) {
         // gate rows in quads 0-3, the same rows of up in quads 4-7 of the token's eight lanes: a gate lane finishes its
@@ -262,13 +308,13 @@ static int sk_row_tiles(const GemmArgs &a, int rt) {
   for (int s = 0; s < a.nseg; s++) n += (a.seg[s].rows + rw - 1) / rw;
   return n;
 }
-template <int RT, int NTT, int DA, int DB>
+template <int RT, int NTT, int ORD>
 static hipError_t launch_skinny_t(const GemmArgs &a, int nrt, int cus, hipStream_t st) {
   const int nt16 = (a.ntok + 15) / 16, ntk = (nt16 + NTT - 1) / NTT;
   // 8 ntk g workgroups: per XCD g row tiles at a time by every token tile; one to a CU, with equal shares of the row tiles
   const int per = sk_tiles_per_wg(nrt, ntk, cus), g = ((nrt + 7) / 8 + per - 1) / per;
-  const size_t lds = 2ull * kSkWaves * 16 * NTT * (16 * RT + 4) * 4;
-  hipLaunchKernelGGL((k_skinny_q8<RT, NTT, DA, DB>), dim3((unsigned)(8 * ntk * g)), dim3(kSkWaves * 64), lds, st, a, nrt, ntk);
+  const size_t lds = 2ull * kSkWaves * 16 * NTT * (16 * RT + 4) * 4 + (ORD == 1 ? 16 * NTT * 16 * RT * 8 * 4 : 0);
+  hipLaunchKernelGGL((k_skinny_q8<RT, NTT, kSkDepth, kSkDepth, ORD>), dim3((unsigned)(8 * ntk * g)), dim3(kSkWaves * 64), lds, st, a, nrt, ntk);
   return hipGetLastError();
 }
 // The tile shape and the time it is expected to take: a start of ~5 us, then per row tile of a workgroup its rounds and
@@ -289,7 +335,13 @@ double skinny_cost(const GemmArgs &a, int cus, int *rt, int *ntt) {
 hipError_t launch_skinny(const GemmArgs &a, int rt, int ntt, int cus, hipStream_t st) {
   if (a.kind != MK_Q8 || a.ldb % 8 || a.ldb < round_up(a.cols / kQB, 8) || (a.w2 && rt != 2)) return hipErrorInvalidValue;
   const int nrt = sk_row_tiles(a, rt);
-#define QPH_SK(R, N) if (rt == R && ntt == N) return launch_skinny_t<R, N, kSkDepth, kSkDepth>(a, nrt, cus, st);
+  if (a.deal.waves > 0 || a.group_blocks > 0) {   // the decode step's orders: one tile of at most 16 tokens
+    if (a.ntok > 16 || a.nseg > 1 || (a.deal.waves > 0 && (a.group_blocks > 0 || a.deal.ns < 1)) || (a.group_blocks > 0 && a.w2))
+      return hipErrorInvalidValue;
+    if (a.group_blocks > 0) return rt == 1 ? launch_skinny_t<1, 1, 2>(a, nrt, cus, st) : launch_skinny_t<2, 1, 2>(a, sk_row_tiles(a, 2), cus, st);
+    return rt == 1 ? launch_skinny_t<1, 1, 1>(a, nrt, cus, st) : launch_skinny_t<2, 1, 1>(a, sk_row_tiles(a, 2), cus, st);
+  }
+#define QPH_SK(R, N) if (rt == R && ntt == N) return launch_skinny_t<R, N, 0>(a, nrt, cus, st);
   QPH_SK(1, 1) QPH_SK(1, 2) QPH_SK(1, 3) QPH_SK(1, 4) QPH_SK(2, 1) QPH_SK(2, 2) QPH_SK(2, 3) QPH_SK(2, 4)
 #undef QPH_SK
   return hipErrorInvalidValue;

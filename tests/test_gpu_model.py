@@ -337,6 +337,49 @@ def test_prefill_behind_a_long_context_splits(cfg, T, n, split, synth, monkeypat
     orc.close()
 
 
+@pytest.mark.parametrize("cfg,T,awo", [("mini", 0, None), ("mini128", 90, "100"), ("mini128", 40, "0"), ("mini_odd", 250, None),
+                                       ("mini_r7", 240, None), ("mini128", 635, None), ("mini128", 1400, None),
+                                       ("mini_r7", 500, None), ("mini", 960, None), ("c1", 33, None), ("c1", 700, None)])
+def test_prefill_all_batches_equal_decode_steps(cfg, T, awo, synth, monkeypatch):
+    """prefill_all of a q8 model in batches: the logits of every token and the cache rows equal the decode steps' bit for
+    bit (QPH_VERIFY_STEPS) - behind short contexts (the fused attention + wo kernels' orders), across the fused limit
+    (640 positions, 100 forced, 256 for mini_r7) in one call, at one split, under 16 splits and at 16 and more (960: the
+    first context that merges in its own launch is inside the call), 1, 2, 16 and 37 tokens (batches of 16 and a rest)"""
+    if awo is not None:
+        monkeypatch.setenv("QPH_AWO_MAX", awo)
+    path = synth(cfg)
+    shape = qa.CONFIGS[cfg]
+    kvd = shape.kv_heads * shape.head_dim
+    rng = np.random.default_rng(T + 3)
+    gpu = qa.HipLlama.load(path, max_ctx=max(T + 64, 300))
+    if T:
+        k = rng.standard_normal((shape.layers, T, kvd)).astype(np.float16)
+        v = rng.standard_normal((shape.layers, T, kvd)).astype(np.float16)
+        gpu.restore(kv_snapshot(k, v))
+    for n in (37, 2, 16, 1):
+        toks = rng.integers(0, shape.vocab, n).astype(np.int32)
+        out = []
+        for steps in (True, False):
+            if steps:
+                monkeypatch.setenv("QPH_VERIFY_STEPS", "1")
+            else:
+                monkeypatch.delenv("QPH_VERIFY_STEPS")
+            print(f"{cfg}: prefill_all of {n} behind {T}, {'steps' if steps else 'batches'}", flush=True)
+            assert gpu.rewind(T)
+            out.append((gpu.prefill_all(toks), gpu.snapshot()))
+            assert gpu.pos() == T + n
+        for i in range(n):
+            np.testing.assert_array_equal(out[0][0][i], out[1][0][i], err_msg=f"token {i} at position {T + i}")
+        assert out[0][1] == out[1][1], "cache rows differ"
+    # a bad id: the tokens before it are fed, then the error, as with steps
+    assert gpu.rewind(T)
+    bad = np.array([1, 2, 3, shape.vocab, 4], np.int32)
+    with pytest.raises(qa.QphError, match="out of range"):
+        gpu.prefill_all(bad)
+    assert gpu.pos() == T + 3
+    gpu.close()
+
+
 def kv_snapshot(k, v):
     """a snapshot in the reference layout (model_llama.cpp:55-63) from per-layer fp16 K / V rows [L][pos][kvd]"""
     pos = k.shape[1]
