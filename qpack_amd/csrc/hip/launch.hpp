@@ -189,15 +189,16 @@ struct PfQuantArgs {
   // bytes apart) the 16-column piece p of each 128-column block (2048 bytes) of token t at byte
   // 1024 (p % 2) + 256 (p / 2) + 16 (t % 16)
   int8_t *th, *tl;
-  // optional: q as two fp16 planes (hi = 256 (q >> 8), lo = q & 255) in the order the q4 / q1 products read them
-  // (k_half), fkind MK_Q4 or MK_Q1: per 16-token tile and 128-column block four 32-column steps x two planes x 1 KiB,
-  // lane 16 lg + t % 16 of step s holding the columns its weight fragment holds
+  // optional: q as two planes in the order the q4 / q1 products read them (k_lowbit).  fkind MK_Q4: halves, hi = 256 (q >>
+  // 8) and lo = q & 255, per 16-token tile and 128-column block four 32-column steps x two planes x 1 KiB; MK_Q1: bytes,
+  // hi = q >> 8 and lo = (q & 255) - 128, two 64-column steps x two planes x 1 KiB.  Lane 16 lg + t % 16 of step s holds the
+  // columns its weight fragment holds
   uint16_t *fp; int fkind;
 };
 hipError_t launch_pf_quant(int pro, const PfQuantArgs &a, int B, hipStream_t st);
 // Y[t][r] = the row's dot product with token t's quantised activation (+ bias[r]), or Y[t][r] += that when resid.
 //   kind MK_Q8: w int8 [rows][cols], scale f32 [rows], wsum = row sums per 128-column block [rows][ldw] (launch_rowsum_q8)
-//   kind MK_Q4 / MK_Q1: w as stored, the scales block-major in st, the activation's fp16 planes fp
+//   kind MK_Q4 / MK_Q1: w as stored, the scales block-major in st, the activation's planes fp in the kind's order
 // one matrix of a multi-matrix product launch (GemmArgs::nseg > 1): its own weights, scales, bias and output
 struct GemmSeg {
   const int8_t *w; const float *scale; const int *wsum; const uint16_t *st;
@@ -210,7 +211,7 @@ struct GemmArgs {
   const int *wsum;   // q8: 128 x the row sums per 128-column block (k_rowsum_q8), [cols / 128][ws_pitch(rows)]
   const int8_t *xh, *xl; const float *xb; int ntok, ldq, ldb;
   const int8_t *th, *tl;   // optional (q8): the planes in 16-token tiles (PfQuantArgs::th), whole tiles allocated
-  // q4 / q1: the activation's fp16 planes (PfQuantArgs::fp), the scales block-major (launch_scale_blocks; st2 of w2)
+  // q4 / q1: the activation's planes (PfQuantArgs::fp, of this kind), the scales block-major (launch_scale_blocks; st2 of w2)
   const uint16_t *fp, *st, *st2;
   const float *xbt; int ldbt;   // q8: the block scales again, block-major [cols / 128][ldbt] (ldbt % 4 == 0, >= ntok)
   float *y; int ldy;
@@ -248,7 +249,7 @@ bool gemm_wants_tiles(const GemmArgs &a);
 // whether launch_gemm runs this q8 launch on the 32 x 32 kernel (the one that can quantise a SwiGLU pair's output)
 bool gemm_uses_32x32(const GemmArgs &a);
 // q4 / q1 products on the f16 matrix cores (skinny.hip): 16 rt rows (8 of each matrix of a pair) x 16 ntt tokens a tile
-hipError_t launch_half(const GemmArgs &a, int cus, hipStream_t st);
+hipError_t launch_lowbit(const GemmArgs &a, int cus, hipStream_t st);
 // scales [rows][G] -> [block][row][4] (q4) or [block][row] (q1)
 hipError_t launch_scale_blocks(int kind, const uint16_t *sc, int rows, int cols, uint16_t *out, hipStream_t st);
 // q8 products of few tokens or few rows (skinny.hip): K split over the waves of a workgroup of 16 rt rows (16 of each

@@ -536,11 +536,11 @@ void HipLlama::prefill_batched(const int *toks, int n) {
   const int d = cfg_.hidden, ff = cfg_.ffn, nb_ld = pf_ldb_;
   const float eps = cfg_.rms_eps;
   // the products of one activation, first planned (which planes does each read), then quantised for, then launched
-  struct Planes { bool rows, tiles; int half; };   // half: MK_Q4 or MK_Q1, whose fragments the fp16 planes match
+  struct Planes { bool rows, tiles; int lowbit; };   // lowbit: MK_Q4 or MK_Q1, whose fragments the planes pf_fp_ match
   auto plan = [&](GemmArgs *g, int ng) {
     Planes p{false, false, 0};
     for (int i = 0; i < ng; i++) {
-      if (g[i].kind != MK_Q8) { if (!p.half) p.half = g[i].kind; }
+      if (g[i].kind != MK_Q8) { if (!p.lowbit) p.lowbit = g[i].kind; }
       else if (gemm_wants_tiles(g[i])) { g[i].th = pf_th_; g[i].tl = pf_tl_; p.tiles = true; }
       else p.rows = true;
     }
@@ -550,7 +550,7 @@ void HipLlama::prefill_batched(const int *toks, int n) {
     PfQuantArgs a{}; a.x = x; a.ldx = ldx; a.norm_w = w; a.eps = eps; a.cols = cols;
     if (p.rows) { a.xh = pf_xh_; a.xl = pf_xl_; }
     if (p.tiles) { a.th = pf_th_; a.tl = pf_tl_; }
-    if (p.half) { a.fp = pf_fp_; a.fkind = p.half; }
+    if (p.lowbit) { a.fp = pf_fp_; a.fkind = p.lowbit; }
     a.ldq = pf_ldq_; a.xb = pf_xb_; a.ldb = nb_ld;
     a.xbt = pf_xbt_; a.ldbt = pf_ldbt_;
     QPH_CK(launch_pf_quant(pro, a, B, st_));
@@ -560,7 +560,7 @@ void HipLlama::prefill_batched(const int *toks, int n) {
     Planes p = plan(g, ng);
     quant(pro, x, ldx, w, cols, B, p);
     for (int i = 0; i < ng; i++) {
-      if (g[i].kind != MK_Q8 && g[i].kind != p.half) { p = Planes{false, false, g[i].kind}; quant(pro, x, ldx, w, cols, B, p); }
+      if (g[i].kind != MK_Q8 && g[i].kind != p.lowbit) { p = Planes{false, false, g[i].kind}; quant(pro, x, ldx, w, cols, B, p); }
       QPH_CK(launch_gemm(g[i], st_));
     }
   };

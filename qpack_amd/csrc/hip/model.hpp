@@ -150,7 +150,7 @@ class HipLlama {
   int pf_ldb_ = 0;                               // row pitch of the block scales
   int8_t *pf_xh2_ = nullptr, *pf_xl2_ = nullptr;   // second planes: the SwiGLU output quantised by the gate / up store
   float *pf_xb2_ = nullptr, *pf_xbt2_ = nullptr;
-  uint16_t *pf_fp_ = nullptr;   // fp16 planes (PfQuantArgs::fp), for models with q4 or q1 layers
+  uint16_t *pf_fp_ = nullptr;   // the q4 / q1 products' planes (PfQuantArgs::fp), for models with such layers
   int *pf_tok_ = nullptr;
   void prefill_batched(const int *toks, int n);
   // prefill_all in batches of up to kVerify tokens whose every logit equals its decode step's bit for bit (q8 models)

@@ -56,25 +56,31 @@ __global__ __launch_bounds__(1024) void k_pf_quant(PfQuantArgs a) {
       *(uint4 *)(a.th + ttile + o) = h; *(uint4 *)(a.tl + ttile + o) = l;
     }
   }
-  if (a.fp)   // fp16 planes: 8 columns of one step's lane per thread
+  if (a.fp && a.fkind == MK_Q4)   // fp16 planes: 8 columns of one step's lane per thread
     for (int i = threadIdx.x; i < cols / 8; i += blockDim.x) {
-      const int b = i >> 4, s = (i >> 2) & 3, lg = i & 3;
-      const int c = b * kQB + (a.fkind == MK_Q1 ? 32 * lg + 4 * s : 32 * s + 4 * lg);   // columns c .. c + 3 and c + 16 ..
+      const int b = i >> 4, s = (i >> 2) & 3, lg = i & 3, c = b * kQB + 32 * s + 4 * lg;   // columns c .. c + 3 and c + 16 ..
       const uint32_t h0 = *(const uint32_t *)(av.xh + c), h1 = *(const uint32_t *)(av.xh + c + 16);
       const uint32_t l0 = *(const uint32_t *)(av.xl + c), l1 = *(const uint32_t *)(av.xl + c + 16);
       auto hi = [](uint32_t w, int k) { return (uint32_t)float_to_half_bits((float)(256 * (int)(int8_t)(w >> (8 * k)))); };
       auto lo = [](uint32_t w, int k) { return (uint32_t)float_to_half_bits((float)((w >> (8 * k)) & 255u)); };
-      uint4 H, L;
-      if (a.fkind == MK_Q1) {
-        H = make_uint4(hi(h0, 0) | hi(h1, 0) << 16, hi(h0, 1) | hi(h1, 1) << 16, hi(h0, 2) | hi(h1, 2) << 16, hi(h0, 3) | hi(h1, 3) << 16);
-        L = make_uint4(lo(l0, 0) | lo(l1, 0) << 16, lo(l0, 1) | lo(l1, 1) << 16, lo(l0, 2) | lo(l1, 2) << 16, lo(l0, 3) | lo(l1, 3) << 16);
-      } else {
-        H = make_uint4(hi(h0, 0) | hi(h0, 2) << 16, hi(h1, 0) | hi(h1, 2) << 16, hi(h0, 1) | hi(h0, 3) << 16, hi(h1, 1) | hi(h1, 3) << 16);
-        L = make_uint4(lo(l0, 0) | lo(l0, 2) << 16, lo(l1, 0) | lo(l1, 2) << 16, lo(l0, 1) | lo(l0, 3) << 16, lo(l1, 1) | lo(l1, 3) << 16);
-      }
       char *o = (char *)a.fp + ((size_t)(t >> 4) * nb + b) * 8192 + 2048 * s + 16 * (16 * lg + (t & 15));
-      *(uint4 *)o = H;
-      *(uint4 *)(o + 1024) = L;
+      *(uint4 *)o = make_uint4(hi(h0, 0) | hi(h0, 2) << 16, hi(h1, 0) | hi(h1, 2) << 16, hi(h0, 1) | hi(h0, 3) << 16, hi(h1, 1) | hi(h1, 3) << 16);
+      *(uint4 *)(o + 1024) = make_uint4(lo(l0, 0) | lo(l0, 2) << 16, lo(l1, 0) | lo(l1, 2) << 16, lo(l0, 1) | lo(l0, 3) << 16, lo(l1, 1) | lo(l1, 3) << 16);
+    }
+  if (a.fp && a.fkind == MK_Q1)   // int8 planes: 16 columns of one step's lane per thread
+    for (int i = threadIdx.x; i < cols / 16; i += blockDim.x) {
+      const int b = i >> 3, s = (i >> 2) & 1, lg = i & 3, c = b * kQB + 32 * lg + 4 * s;   // columns c + 8 j + 0..3, j = 0..3
+      char *o = (char *)a.fp + ((size_t)(t >> 4) * nb + b) * 4096 + 2048 * s + 16 * (16 * lg + (t & 15));
+      auto put = [&](const int8_t *x, uint32_t flip, char *out) {   // a 4 x 4 transpose of bytes
+        const uint32_t d0 = *(const uint32_t *)(x + c) ^ flip, d1 = *(const uint32_t *)(x + c + 8) ^ flip;
+        const uint32_t d2 = *(const uint32_t *)(x + c + 16) ^ flip, d3 = *(const uint32_t *)(x + c + 24) ^ flip;
+        auto dword = [&](int k) {
+          return ((d0 >> (8 * k)) & 255u) | ((d1 >> (8 * k)) & 255u) << 8 | ((d2 >> (8 * k)) & 255u) << 16 | ((d3 >> (8 * k)) & 255u) << 24;
+        };
+        *(uint4 *)out = make_uint4(dword(0), dword(1), dword(2), dword(3));
+      };
+      put(av.xh, 0, o);
+      put((const int8_t *)av.xl, 0x80808080u, o + 1024);   // lo - 128
     }
   for (int b = threadIdx.x; b < nb; b += blockDim.x) a.xb[(size_t)t * a.ldb + b] = av.bs[b];
   if (a.xbt)
@@ -803,7 +809,7 @@ hipError_t launch_gemm(const GemmArgs &a0, hipStream_t st) {
     }
   } else if (a.kind == MK_Q4 || a.kind == MK_Q1) {
     if (!a.st) return hipErrorInvalidValue;
-    return launch_half(a, gemm_cus(), st);
+    return launch_lowbit(a, gemm_cus(), st);
   } else {
     return hipErrorInvalidValue;
   }

@@ -347,25 +347,30 @@ hipError_t launch_skinny(const GemmArgs &a, int rt, int ntt, int cus, hipStream_
   return hipErrorInvalidValue;
 }
 
-// ------------------------------------------------------------------ q4 and q1 weights on the f16 matrix cores
-// A q4 group (32 columns) is a dot product of 4-bit integers with 16-bit ones: at most 8 x 32 x 32767 < 2^23 in size, so
-// v_mfma_f32_16x16x32_f16 gives it exactly, as a float: the weights n = nibble - 8 are exact halves, the activation goes in
-// as two halves q = hi + lo (hi = 256 (q >> 8), lo = q & 255), every product and partial sum is an integer below 2^24.
-// What is left for the vector ALU is one fma per output and group, with the group's fp16 scale; on the int8 cores it is a
-// shift-add, a conversion and an fma, and the offset corrections.  A q1 group (128 columns) is below 2^22 likewise.
+// ------------------------------------------------------------------ q4 and q1 weights
+// q4 on the f16 matrix cores: a group (32 columns) is a dot product of 4-bit integers with 16-bit ones, at most 8 x 32 x
+// 32767 < 2^23 in size, so v_mfma_f32_16x16x32_f16 gives it exactly, as a float: the weights n = nibble - 8 are exact
+// halves, the activation goes in as two halves q = hi + lo (hi = 256 (q >> 8), lo = q & 255), every product and partial sum
+// is an integer below 2^24.  What is left for the vector ALU is one fma per output and group, with the group's fp16 scale;
+// on the int8 cores it is a shift-add, a conversion and an fma, and the offset corrections.
 //   blk = sum over the block's groups of scale * sum, acc = fma(bs[token][block], blk, acc)
+// q1 on the int8 matrix cores, which do twice the columns in the time: a group is a whole block (128 columns, two steps),
+// so the integer work after it is a fourth of q4's.  A bit becomes the byte +-64 (0x40 or 0xc0: a shift, a mask and an
+// or for four); with T = 32 sum(W) + the hi plane, 256 T + the plane lo - 128 = 64 times the group's sum, exact in int32 and as a
+// float (the sum is below 2^22), and 1 / 64 goes into the scale.  64 sum(W) is one more product, with a constant plane.
 // Tile: 16 RT rows x 16 NTT tokens per workgroup; its 8 waves take every eighth block each, add no barrier until the tile's
-// end, and their fp32 partials are summed there in wave order through LDS.
+// end, and their fp32 partials are summed there in wave order through LDS, 32 tokens at a time.
 // Operands: weights from HBM to registers as stored.  q4: lane l loads the 16 bytes of group l / 16 of row l % 16; a 4 x 4
 // transpose of dwords over the four 16-lane rows (permlane swaps) gives every lane dword l / 16 of each group, and a dword
-// becomes four half pairs with a mask, 0x6400 (1024 + nibble) and one packed subtraction.  q1: dword l / 16 of the block; a
-// shift and a bit-field insert turn two bits into +-1.  Activations in the order these fragments have (PfQuantArgs::fp: 1
-// KiB of consecutive bytes each), straight from L2 to registers, one block ahead (64 rows by 48 tokens, or 32 by 64, spill
-// with q4: 2 to 4 times slower).  The rows' scales of a block (512 bytes,
-// one load) are handed to the lanes through LDS, the tokens' block scales stay in LDS from the start.
+// becomes four half pairs with a mask, 0x6400 (1024 + nibble) and one packed subtraction.  q1: dword l / 16 of the block.
+// Activations in the order these fragments have (PfQuantArgs::fp: 1 KiB of consecutive bytes each), straight from L2 to
+// registers, one block ahead (q4 with 64 rows by 48 tokens, or 32 by 64, spills: 2 to 4 times slower).  The rows' scales of
+// a block (one load) are handed to the lanes through LDS, the tokens' block scales stay in LDS from the start.
 // Measured (MI355X, weights from HBM, us; before: 128 x 128 tiles on the int8 cores): q4 3584 x 18944 at 150 tokens 780 ->
-// 99, 18944 x 3584 255 -> 71, 896 x 4864 at 512 tokens 164 -> 20.  A block of a 64 x 32 tile is 64 MFMAs and ~330 vector
-// instructions per wave; without any loads 150 tokens of 18944 x 3584 take 9 % less: their issue bounds it, ahead of L2.
+// 99, 18944 x 3584 255 -> 71, 896 x 4864 at 512 tokens 164 -> 20.  37888 x 3584 at 512 tokens take 244 us: with the two
+// planes 1.14 POP/s, what a large bf16 matrix product reaches here (1.12 PFLOP/s).  Without any loads 150 tokens of 18944 x
+// 3584 take 9 % less, without the unpacking and the scaling 5 %, with one plane 15 %: no single resource is left to relieve.
+// q1 at 300 tokens (before: on the f16 cores like q4) 28672 x 4096 200 -> 119, 4096 x 14336 116 -> 72.
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef _Float16 h4v __attribute__((ext_vector_type(4)));
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
@@ -390,24 +395,27 @@ __device__ __forceinline__ h8v q4_half8(uint32_t w, uint32_t c1, uint32_t c2) {
   const uint32_t p3 = bits(__builtin_bit_cast(h2v, (v & 0x00f000f0u) | c2) - o2);
   return __builtin_bit_cast(h8v, make_uint4(p0, p1, p2, p3));
 }
-// step s of a q1 dword: halves (bit 4 s + j, bit 16 + 4 s + j), j = 0..3, as -1 (set) or +1
-__device__ __forceinline__ h8v q1_half8(uint32_t w, int s) {
+// step s of a q1 dword: bytes (bits 4 s + j of its four bytes), j = 0..3, as -64 (set) or +64: they differ in the sign bit only
+__device__ __forceinline__ v4i q1_bytes16(uint32_t w, int s, uint32_t c) {
   uint32_t p[4];
 #pragma unroll
-  for (int j = 0; j < 4; j++) p[j] = ((w << (15 - 4 * s - j)) & 0x80008000u) | 0x3c003c00u;
-  return __builtin_bit_cast(h8v, make_uint4(p[0], p[1], p[2], p[3]));
+  for (int j = 0; j < 4; j++) p[j] = ((w << (7 - 4 * s - j)) & 0x80808080u) | c;
+  return __builtin_bit_cast(v4i, make_uint4(p[0], p[1], p[2], p[3]));
 }
 
 template <int KIND, int RT, int NTT>
-__global__ __launch_bounds__(kSkWaves * 64) void k_half(GemmArgs a, int nrt, int ntk, int tg, int rg) {
+__global__ __launch_bounds__(kSkWaves * 64) void k_lowbit(GemmArgs a, int nrt, int ntk, int tg, int rg) {
   constexpr bool Q4 = KIND == MK_Q4;
   constexpr int RW = 16 * RT, NT = 16 * NTT, P = RW + 4, SB = Q4 ? 8 : 2;   // SB: scale bytes per row and block
+  constexpr int NS = Q4 ? 4 : 2, BB = NS * 2048;                            // MFMA steps and activation bytes per block
+  typedef typename std::conditional<Q4, h8v, v4i>::type frag_t;
   extern __shared__ __align__(16) char hsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
   const int nb = a.cols / kQB;
-  float *red = (float *)hsm;                                  // [8 waves][NT][P] partials
-  char *scl = hsm + (size_t)kSkWaves * NT * P * 4 + wave * (RW * SB);   // this wave's block scales [RW][SB]
-  float *bsl = (float *)(hsm + (size_t)kSkWaves * (NT * P * 4 + RW * SB));   // [nb][NT]
+  constexpr int RN = NTT < 2 ? NTT : 2, RT16 = 16 * RN;       // token tiles whose partials are summed at a time
+  float *red = (float *)hsm;                                  // [8 waves][16 RN][P] partials
+  char *scl = hsm + (size_t)kSkWaves * RT16 * P * 4 + wave * (RW * SB);   // this wave's block scales [RW][SB]
+  float *bsl = (float *)(hsm + (size_t)kSkWaves * (RT16 * P * 4 + RW * SB));   // [nb][NT]
   const bool paired = a.w2 != nullptr;   // the tile's first RW / 2 rows from the gate matrix, the others the same rows of up
   // token tile tk and row tiles rt0, rt0 + rts, ...: the XCD's workgroups are dealt in sets of tg token tiles x rg row tiles
   const int q = (int)blockIdx.x >> 3, in_set = q % (tg * rg);
@@ -475,15 +483,13 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_half(GemmArgs a, int nrt, int
   const int nt16 = (a.ntok + 15) / 16;
   const char *fb[NTT];
 #pragma unroll
-  for (int n = 0; n < NTT; n++) fb[n] = (const char *)a.fp + (size_t)min(tk * NTT + n, nt16 - 1) * nb * 8192 + 16 * lane;
+  for (int n = 0; n < NTT; n++) fb[n] = (const char *)a.fp + (size_t)min(tk * NTT + n, nt16 - 1) * nb * BB + 16 * lane;
   int bj = 0;
-  h8v B[4][NTT][2];
-  auto load_b = [&](int s) {
-    const size_t o = (size_t)min(wave + kSkWaves * bj, nb - 1) * 8192 + 2048 * s;
+  frag_t B[NS][NTT][2];
+  auto load_b = [&](int s, int n) {
+    const char *p = fb[n] + (size_t)min(wave + kSkWaves * bj, nb - 1) * BB + 2048 * s;
 #pragma unroll
-    for (int n = 0; n < NTT; n++)
-#pragma unroll
-      for (int pl = 0; pl < 2; pl++) B[s][n][pl] = *(const h8v *)(fb[n] + o + 1024 * pl);
+    for (int pl = 0; pl < 2; pl++) B[s][n][pl] = *(const frag_t *)(p + 1024 * pl);
   };
 
   f4v acc[RT][NTT];
@@ -496,12 +502,14 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_half(GemmArgs a, int nrt, int
   zero();
   raw_t A[RT];
   scr_t S;
-  uint32_t c1 = 0x64006400u, c2 = 0x54005400u;
+  uint32_t c1 = Q4 ? 0x64006400u : 0x40404040u, c2 = 0x54005400u;
   asm volatile("" : "+v"(c1), "+v"(c2));
   w_tile();
   load_w(A, S);
 #pragma unroll
-  for (int s = 0; s < 4; s++) load_b(s);
+  for (int s = 0; s < NS; s++)
+#pragma unroll
+    for (int n = 0; n < NTT; n++) load_b(s, n);
   bj = nj > 1 ? 1 : 0;
   __syncthreads();   // the block scales
 
@@ -539,79 +547,119 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_half(GemmArgs a, int nrt, int
     float bs[NTT];
 #pragma unroll
     for (int n = 0; n < NTT; n++) bs[n] = bsl[b * NT + 16 * n + lr];
-    f4v blk[RT][NTT];
+    if constexpr (Q4) {
+      f4v blk[RT][NTT];
 #pragma unroll
-    for (int s = 0; s < 4; s++) {
-      h8v F[RT];
+      for (int s = 0; s < 4; s++) {
+        h8v F[RT];
 #pragma unroll
-      for (int i = 0; i < RT; i++) F[i] = Q4 ? q4_half8(q[i][s], c1, c2) : q1_half8(q[i][0], s);
+        for (int i = 0; i < RT; i++) F[i] = q4_half8(q[i][s], c1, c2);
 #pragma unroll
-      for (int n = 0; n < NTT; n++)
+        for (int n = 0; n < NTT; n++)
+#pragma unroll
+          for (int i = 0; i < RT; i++) {
+            f4v T = (f4v){0.f, 0.f, 0.f, 0.f};
+            T = __builtin_amdgcn_mfma_f32_16x16x32_f16(F[i], B[s][n][0], T, 0, 0, 0);
+            T = __builtin_amdgcn_mfma_f32_16x16x32_f16(F[i], B[s][n][1], T, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const float w = (float)sc[i][r][s];
+              blk[i][n][r] = s == 0 ? w * T[r] : __builtin_fmaf(w, T[r], blk[i][n][r]);
+            }
+          }
+#pragma unroll
+        for (int n = 0; n < NTT; n++) load_b(s, n);
+      }
+#pragma unroll
+      for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int n = 0; n < NTT; n++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(bs[n], blk[i][n][r], acc[i][n][r]);
+    } else {
+      v4i F[2][RT], R[RT];
+      const v4i ones = (v4i){0x01010101, 0x01010101, 0x01010101, 0x01010101};
+#pragma unroll
+      for (int i = 0; i < RT; i++) {
+        R[i] = (v4i){0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          F[s][i] = q1_bytes16(q[i][0], s, c1);
+          R[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(F[s][i], ones, R[i], 0, 0, 0);
+        }
+      }
+      float w[RT][4];
+#pragma unroll
+      for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) { R[i][r] >>= 1; w[i][r] = -0.015625f * (float)sc[i][0][r]; }
+#pragma unroll
+      for (int n = 0; n < NTT; n++) {
+        v4i T[RT];
 #pragma unroll
         for (int i = 0; i < RT; i++) {
-          f4v T = (f4v){0.f, 0.f, 0.f, 0.f};
-          if (!Q4 && s > 0) T = blk[i][n];   // q1: one sum for the block
-          T = __builtin_amdgcn_mfma_f32_16x16x32_f16(F[i], B[s][n][0], T, 0, 0, 0);
-          T = __builtin_amdgcn_mfma_f32_16x16x32_f16(F[i], B[s][n][1], T, 0, 0, 0);
-          if (!Q4) { blk[i][n] = T; continue; }
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const float w = (float)sc[i][r][s];
-            blk[i][n][r] = s == 0 ? w * T[r] : __builtin_fmaf(w, T[r], blk[i][n][r]);
-          }
+          T[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(F[0][i], B[0][n][0], R[i], 0, 0, 0);
+          T[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(F[1][i], B[1][n][0], T[i], 0, 0, 0);
         }
-      load_b(s);
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) T[i][r] = (int)((uint32_t)T[i][r] << 8);
+          T[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(F[0][i], B[0][n][1], T[i], 0, 0, 0);
+          T[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(F[1][i], B[1][n][1], T[i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; s++) load_b(s, n);
+#pragma unroll
+        for (int i = 0; i < RT; i++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(bs[n], w[i][r] * (float)T[i][r], acc[i][n][r]);
+      }
     }
-#pragma unroll
-    for (int i = 0; i < RT; i++)
-#pragma unroll
-      for (int n = 0; n < NTT; n++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const float v = Q4 ? blk[i][n][r] : -(float)sc[i][0][r] * blk[i][n][r];
-          acc[i][n][r] = __builtin_fmaf(bs[n], v, acc[i][n][r]);
-        }
     bj = bj + 1 < nj ? bj + 1 : 0;
   };
 
   for (int tile = 0; tile < mine; tile++) {
     for (int j = 0; j < nj; j++) block(wave + kSkWaves * j);
-#pragma unroll
-    for (int i = 0; i < RT; i++)
-#pragma unroll
-      for (int n = 0; n < NTT; n++)
-        *(f4v *)(red + (wave * NT + 16 * n + lr) * P + 16 * i + 4 * lg) = acc[i][n];
-    zero();
-    lds_barrier();
     const Tile t = tile_of(rt0 + tile * rts);
-    auto sum = [&](int tok, int row) {
-      f4v v = *(const f4v *)(red + tok * P + row);
 #pragma unroll
-      for (int w = 1; w < kSkWaves; w++) v += *(const f4v *)(red + (w * NT + tok) * P + row);
-      return v;
-    };
-    const int quads = paired ? RW / 8 : RW / 4;
-    for (int e = tid; e < NT * quads; e += kSkWaves * 64) {
-      const int tok = e / quads, cq = e % quads, gt = tk * NT + tok, row = t.r0 + 4 * cq;
-      if (gt >= a.ntok) continue;
-      f4v v = sum(tok, 4 * cq);
-      float *yt = t.y + (size_t)gt * t.ldy;
-      if (paired) {
-        const f4v u = sum(tok, RW / 2 + 4 * cq);
+    for (int n0 = 0; n0 < NTT; n0 += RN) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) v[r] = sk_silu_mul(v[r], u[r]);
+      for (int n = n0; n < n0 + RN && n < NTT; n++)
+#pragma unroll
+        for (int i = 0; i < RT; i++)
+          *(f4v *)(red + (wave * RT16 + 16 * (n - n0) + lr) * P + 16 * i + 4 * lg) = acc[i][n];
+      lds_barrier();
+      auto sum = [&](int tok, int row) {
+        f4v v = *(const f4v *)(red + tok * P + row);
+#pragma unroll
+        for (int w = 1; w < kSkWaves; w++) v += *(const f4v *)(red + (w * RT16 + tok) * P + row);
+        return v;
+      };
+      const int quads = paired ? RW / 8 : RW / 4, ntoks = NTT - n0 < RN ? 16 * (NTT - n0) : RT16;
+      for (int e = tid; e < ntoks * quads; e += kSkWaves * 64) {
+        const int tok = e / quads, cq = e % quads, gt = tk * NT + 16 * n0 + tok, row = t.r0 + 4 * cq;
+        if (gt >= a.ntok) continue;
+        f4v v = sum(tok, 4 * cq);
+        float *yt = t.y + (size_t)gt * t.ldy;
+        if (paired) {
+          const f4v u = sum(tok, RW / 2 + 4 * cq);
+#pragma unroll
+          for (int r = 0; r < 4; r++) v[r] = sk_silu_mul(v[r], u[r]);
+        }
+        if (row + 3 < t.rows && (t.ldy & 3) == 0) {
+          if (a.resid) v += *(const f4v *)(yt + row);
+          else if (t.bias) v += *(const f4v *)(t.bias + row);
+          *(f4v *)(yt + row) = v;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            if (row + r < t.rows) yt[row + r] = a.resid ? yt[row + r] + v[r] : t.bias ? v[r] + t.bias[row + r] : v[r];
+        }
       }
-      if (row + 3 < t.rows && (t.ldy & 3) == 0) {
-        if (a.resid) v += *(const f4v *)(yt + row);
-        else if (t.bias) v += *(const f4v *)(t.bias + row);
-        *(f4v *)(yt + row) = v;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          if (row + r < t.rows) yt[row + r] = a.resid ? yt[row + r] + v[r] : t.bias ? v[r] + t.bias[row + r] : v[r];
-      }
+      lds_barrier();
     }
-    lds_barrier();
+    zero();
   }
 }
 
@@ -633,14 +681,14 @@ hipError_t launch_scale_blocks(int kind, const uint16_t *sc, int rows, int cols,
 // token tiles in sets of tg: the workgroups on the chip at a time share a set's activations, which then stay in the XCDs'
 // L2 while the weights stream past (18944 x 3584, 2048 tokens: one set of 64 tiles 1194 us, sets of 16 / 8 / 4 / 2
 // 919 / 865 / 861 / 910; up to 16 tiles one set is as fast)
-static void half_sets(int ntk, int *sets, int *tg) {
+static void lowbit_sets(int ntk, int *sets, int *tg) {
   const int cap = ntk <= 16 ? 16 : 8;
   *sets = (ntk + cap - 1) / cap; *tg = (ntk + *sets - 1) / *sets;
 }
-static size_t half_lds(int kind, int rt, int ntt, int nb) {
-  return (size_t)kSkWaves * (16 * ntt * (16 * rt + 4) * 4 + 16 * rt * (kind == MK_Q4 ? 8 : 2)) + (size_t)nb * 16 * ntt * 4;
+static size_t lowbit_lds(int kind, int rt, int ntt, int nb) {
+  return (size_t)kSkWaves * (16 * std::min(ntt, 2) * (16 * rt + 4) * 4 + 16 * rt * (kind == MK_Q4 ? 8 : 2)) + (size_t)nb * 16 * ntt * 4;
 }
-static int half_row_tiles(const GemmArgs &a, int rt) {
+static int lowbit_row_tiles(const GemmArgs &a, int rt) {
   const int rw = a.w2 ? 8 * rt : 16 * rt;
   if (a.nseg < 2) return (a.rows + rw - 1) / rw;
   int n = 0;
@@ -648,42 +696,47 @@ static int half_row_tiles(const GemmArgs &a, int rt) {
   return n;
 }
 template <int KIND, int RT, int NTT>
-static hipError_t launch_half_t(const GemmArgs &a, int cus, hipStream_t st) {
-  const int nrt = half_row_tiles(a, RT), nt16 = (a.ntok + 15) / 16, ntk = (nt16 + NTT - 1) / NTT;
+static hipError_t launch_lowbit_t(const GemmArgs &a, int cus, hipStream_t st) {
+  const int nrt = lowbit_row_tiles(a, RT), nt16 = (a.ntok + 15) / 16, ntk = (nt16 + NTT - 1) / NTT;
   int sets, tg;
-  half_sets(ntk, &sets, &tg);
+  lowbit_sets(ntk, &sets, &tg);
   const int per = sk_tiles_per_wg(nrt, tg, cus), rg = ((nrt + 7) / 8 + per - 1) / per;
-  const size_t lds = half_lds(KIND, RT, NTT, a.cols / kQB);
+  const size_t lds = lowbit_lds(KIND, RT, NTT, a.cols / kQB);
   if (lds > 160 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_half<KIND, RT, NTT>), dim3((unsigned)(8 * sets * tg * rg)), dim3(kSkWaves * 64), lds, st, a, nrt, ntk, tg, rg);
+  hipLaunchKernelGGL((k_lowbit<KIND, RT, NTT>), dim3((unsigned)(8 * sets * tg * rg)), dim3(kSkWaves * 64), lds, st, a, nrt, ntk, tg, rg);
   return hipGetLastError();
 }
-// The tile shape for a launch: a start of ~5 us, then per row tile of a workgroup every wave's blocks and ~1 us for its
-// end (block times with every CU busy, from the shapes above).  32-row tiles where 64-row ones leave CUs idle.
-static void half_tile(const GemmArgs &a, int cus, int *rt, int *ntt) {
-  static const int shape[4][2] = {{2, 1}, {2, 2}, {4, 1}, {4, 2}};
-  static const double block_us[4] = {1.55, 2.0, 2.1, 2.45};
+// The tile shape for a launch: a start of ~5 us, then per row tile of a workgroup every wave's blocks and ~1 us for each
+// pass of its end (block times with every CU busy, fitted to the shapes above, within 10 % of what they take).  32-row
+// tiles where 64-row ones leave CUs idle; 64 tokens for q1 where there are enough tiles (28672 x 4096 at 512 tokens: 32
+// tokens a tile 219 us, 64 178; 4096 x 14336 at 50 tokens: 64 x 64 37 us, 32 x 32 20.5).
+static void lowbit_tile(const GemmArgs &a, int cus, int *rt, int *ntt) {
+  static const int shape[5][2] = {{2, 1}, {2, 2}, {4, 1}, {4, 2}, {4, 4}};
+  static const double block_us[2][5] = {{1.55, 2.0, 2.1, 2.45, 0}, {0.65, 1.1, 1.1, 1.63, 2.6}};   // q4, q1
+  const bool q1 = a.kind == MK_Q1;
   const int rounds = (a.cols / kQB + kSkWaves - 1) / kSkWaves, nt16 = (a.ntok + 15) / 16;
   double best = 1e30;
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < (q1 ? 5 : 4); i++) {
     const int ntk = (nt16 + shape[i][1] - 1) / shape[i][1];
     int sets, tg;
-    half_sets(ntk, &sets, &tg);
-    const double c = sets * sk_tiles_per_wg(half_row_tiles(a, shape[i][0]), tg, cus) * (rounds * block_us[i] + 1);
+    lowbit_sets(ntk, &sets, &tg);
+    const double c = sets * sk_tiles_per_wg(lowbit_row_tiles(a, shape[i][0]), tg, cus) * (rounds * block_us[q1][i] + (shape[i][1] + 1) / 2);
     if (c < best) { best = c; *rt = shape[i][0]; *ntt = shape[i][1]; }
   }
 }
-hipError_t launch_half(const GemmArgs &a, int cus, hipStream_t st) {
+hipError_t launch_lowbit(const GemmArgs &a, int cus, hipStream_t st) {
   if ((a.kind != MK_Q4 && a.kind != MK_Q1) || !a.fp || a.ldb < a.cols / kQB || (a.w2 && !a.st2)) return hipErrorInvalidValue;
   int rt, ntt;
-  half_tile(a, cus, &rt, &ntt);
+  lowbit_tile(a, cus, &rt, &ntt);
   if (const char *e = getenv("QPH_SKINNY")) {   // test hook: the tile (two digits, rows / 16 and tokens / 16)
     rt = atoi(e) / 10 >= 4 ? 4 : 2; ntt = std::max(1, std::min(2, atoi(e) % 10));
+    if (a.kind == MK_Q1 && atoi(e) == 44) ntt = 4;
   }
 #define QPH_HF(R, N)                                                      \
   if (rt == R && ntt == N)                                                \
-    return a.kind == MK_Q4 ? launch_half_t<MK_Q4, R, N>(a, cus, st) : launch_half_t<MK_Q1, R, N>(a, cus, st);
+    return a.kind == MK_Q4 ? launch_lowbit_t<MK_Q4, R, N>(a, cus, st) : launch_lowbit_t<MK_Q1, R, N>(a, cus, st);
   QPH_HF(2, 1) QPH_HF(2, 2) QPH_HF(4, 1) QPH_HF(4, 2)
+  if (a.kind == MK_Q1 && rt == 4 && ntt == 4) return launch_lowbit_t<MK_Q1, 4, 4>(a, cus, st);
 #undef QPH_HF
   return hipErrorInvalidValue;
 }

@@ -260,9 +260,10 @@ def test_prefill_few_token_kernel_agrees(cfg, n, synth, monkeypatch):
 
 
 @pytest.mark.parametrize("n", [2, 17, 70, 300])
-@pytest.mark.parametrize("cfg,tile", [("mini_q1", "21"), ("mini_q1", "42"), ("mini_q1m", "22"), ("mini_q1m", "41"), ("mini_q1m", "")])
+@pytest.mark.parametrize("cfg,tile", [("mini_q1", "21"), ("mini_q1", "42"), ("mini_q1m", "22"), ("mini_q1m", "41"), ("mini_q1", "44"), ("mini_q1m", "44"),
+                                      ("mini_q1m", "")])
 def test_batched_prefill_q1(cfg, tile, n, synth, monkeypatch):
-    """prompts of models with q1 MLP matrices go through the batched products (k_half, its tiles forced): logits and every
+    """prompts of models with q1 MLP matrices go through the batched products (k_lowbit, its tiles forced): logits and every
     cache row against the oracle's decode steps and against this library's (QPH_PREFILL_STEPS), the greedy continuation
     against the oracle's up to a near-tie; mini_q1m mixes q1 and q8 down matrices"""
     if tile:
