@@ -47,6 +47,26 @@ def test_topk_ties_and_specials(M):
     check(-np.ones(n, np.float32), M)
 
 
+@pytest.mark.parametrize("n", [65, 1025, 33000, 300000])
+@pytest.mark.parametrize("M", [64, 65, 128, 129, 256, 257, 512])
+@pytest.mark.parametrize("order", ["up", "down", "last", "random"])
+def test_topk_list_edges(n, M, order):
+    """list lengths 64, 128, 256 and 512 at and around their edges, run counts that leave waves without keys, survivors
+    of more than one second-round chunk (300000 values, M = 512: 74 x 512), and inputs whose every run replaces the
+    whole list (ascending), none does (descending), or only the last does"""
+    if M > n:
+        pytest.skip("M <= n")
+    x = np.arange(n, dtype=np.float32)
+    if order == "down":
+        x = x[::-1].copy()
+    elif order == "last":
+        x = np.concatenate([np.zeros(n - M, np.float32), -x[:M] + M])
+    elif order == "random":
+        x = np.random.default_rng(n + M).permutation(x // 3).astype(np.float32)
+    print(f"topk n={n} M={M} {order}", flush=True)
+    check(x, M)
+
+
 def test_topk_rejects_bad_sizes():
     for n, M in ((100, 0), (100, 101), (600, 513)):
         with pytest.raises(qa.QphError):
