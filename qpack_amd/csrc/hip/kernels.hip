@@ -597,6 +597,24 @@ hipError_t launch_embed(const DMat &embed, const Ctl *ctl, float *x, hipStream_t
   return hipGetLastError();
 }
 
+// 16 bytes a thread; bound by the link to the host's memory (~50 GB/s: 512 KiB in ~11 us).  n16, off16, layer16: 16-byte units
+__global__ __launch_bounds__(kThreads) void k_cache_gather(const uint4 *kc, const uint4 *vc, size_t layer16, uint32_t n16, uint32_t row,
+                                                           uint32_t off16, uint32_t len16, uint4 *out) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= len16) return;
+  const uint32_t r = row + (off16 + i) / n16, c = (off16 + i) % n16;   // row r: layer r / 2, its K (even) or V
+  out[i] = (r & 1 ? vc : kc)[(size_t)(r >> 1) * layer16 + c];
+}
+hipError_t launch_cache_gather(const uint16_t *kc, const uint16_t *vc, size_t layer, size_t nb, size_t off, size_t len, void *out,
+                               hipStream_t st) {
+  if (layer % 16 || nb % 16 || off % 16 || len % 16 || !nb || nb + len > ((size_t)1 << 35)) return hipErrorInvalidValue;
+  if (!len) return hipSuccess;
+  const size_t n16 = nb / 16, o16 = off / 16, len16 = len / 16;
+  hipLaunchKernelGGL(k_cache_gather, dim3((unsigned)((len16 + kThreads - 1) / kThreads)), dim3(kThreads), 0, st, (const uint4 *)kc,
+                     (const uint4 *)vc, layer / 16, (uint32_t)n16, (uint32_t)(o16 / n16), (uint32_t)(o16 % n16), (uint32_t)len16, (uint4 *)out);
+  return hipGetLastError();
+}
+
 // out = RMSNorm(x) * w with the PRO_NORM prologue's arithmetic (same inverse norm, same products)
 __global__ __launch_bounds__(1024) void k_rmsnorm(const float *x, const float *w, int n, float eps, float *out) {
   extern __shared__ __align__(16) char smem[];

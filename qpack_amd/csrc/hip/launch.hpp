@@ -241,6 +241,10 @@ size_t gemm_lds_bytes();
 // row pitch of the block-major row sums: rows rounded up to 64 (16-byte loads of 4 rows stay inside a block's run)
 __host__ __device__ inline int ws_pitch(int rows) { return (rows + 63) & ~63; }
 // out[row][block] = sum of W[row] over each 128-column block
+// bytes [off, off + len) of a snapshot's body (per layer the first nb bytes of its K cache, then of its V cache; layers
+// `layer` bytes apart) -> out, which may be pinned host memory.  All sizes are multiples of 16
+hipError_t launch_cache_gather(const uint16_t *kc, const uint16_t *vc, size_t layer, size_t nb, size_t off, size_t len, void *out,
+                               hipStream_t st);
 hipError_t launch_rowsum_q8(const int8_t *w, int rows, int cols, int *out, hipStream_t st);
 // launch_gemm runs a q8 launch with th set on the few-token kernel, others on the tiled ones (which read xh / xl);
 // gemm_wants_tiles: whether th is the faster choice for this product (the pointers need not be set yet)

@@ -231,6 +231,9 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
   QPH_CK(hipHostMalloc((void **)&hctl_, kRing * sizeof(Ctl), hipHostMallocDefault));
   QPH_CK(hipHostMalloc((void **)&hout_, 4ull * std::max(V, d), hipHostMallocDefault));
   QPH_CK(hipHostMalloc((void **)&htok_, 4ull * (ctx_ + 1), hipHostMallocDefault));
+  QPH_CK(hipHostMalloc((void **)&snap_host_, kSnapSlots * kSnapSlot, hipHostMallocDefault));
+  memset(snap_host_, 0, kSnapSlots * kSnapSlot);   // its pages' first touch: about a microsecond each, here and not in a first snapshot
+  for (hipEvent_t &e : snap_ev_) QPH_CK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   QPH_CK(hipHostMalloc((void **)&htopk_, 8ull * kTopkMax, hipHostMallocDefault));
   {
     const size_t keys = topk_scratch_keys(V, std::min(kTopkMax, V));
@@ -259,6 +262,8 @@ HipLlama::~HipLlama() {
   if (htok_) (void)hipHostFree(htok_);
   if (vf_host_) (void)hipHostFree(vf_host_);
   for (hipEvent_t e : vf_ev_) if (e) (void)hipEventDestroy(e);
+  for (hipEvent_t e : snap_ev_) if (e) (void)hipEventDestroy(e);
+  if (snap_host_) (void)hipHostFree(snap_host_);
   if (htopk_) (void)hipHostFree(htopk_);
   if (hstatus_) (void)hipHostFree(hstatus_);
   if (st_) (void)hipStreamDestroy(st_);
@@ -784,9 +789,23 @@ void HipLlama::set_pos(int pos) {
 void HipLlama::snapshot(uint8_t *buf, int64_t cap) {
   if (cap < snapshot_size()) throw std::runtime_error("snapshot buffer too small");
   { QPH_CK(hipStreamSynchronize(st_)); check_status(); }
-  memcpy(buf, &pos_, 4); uint8_t *p = buf + 4; const size_t nb = (size_t)pos_ * kvd_ * 2;
-  for (int l = 0; l < cfg_.layers; l++)
-    for (uint16_t *c : {kc_, vc_}) { QPH_CK(hipMemcpy(p, c + (size_t)l * ctx_ * kvd_, nb, hipMemcpyDeviceToHost)); p += nb; }
+  memcpy(buf, &pos_, 4);
+  // pieces of the snapshot's body gathered into the pinned slots ahead, copied to the caller's memory in turn
+  const size_t nb = (size_t)pos_ * kvd_ * 2, total = 2 * nb * cfg_.layers, pieces = (total + kSnapSlot - 1) / kSnapSlot;
+  auto gather = [&](size_t i) {
+    const size_t o = i * kSnapSlot;
+    QPH_CK(launch_cache_gather(kc_, vc_, (size_t)ctx_ * kvd_ * 2, nb, o, std::min(total - o, kSnapSlot), snap_host_ + i % kSnapSlots * kSnapSlot, st_));
+    QPH_CK(hipEventRecord(snap_ev_[i % kSnapSlots], st_));
+  };
+  try {
+    for (size_t i = 0; i < std::min(pieces, kSnapSlots); i++) gather(i);
+    for (size_t i = 0; i < pieces; i++) {
+      const size_t o = i * kSnapSlot;
+      QPH_CK(hipEventSynchronize(snap_ev_[i % kSnapSlots]));
+      memcpy(buf + 4 + o, snap_host_ + i % kSnapSlots * kSnapSlot, std::min(total - o, kSnapSlot));
+      if (i + kSnapSlots < pieces) gather(i + kSnapSlots);
+    }
+  } catch (...) { (void)hipStreamSynchronize(st_); throw; }
 }
 
 void HipLlama::restore(const uint8_t *buf, int64_t n) {

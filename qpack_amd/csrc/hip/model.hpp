@@ -96,6 +96,12 @@ class HipLlama {
   int *topk_idx_ = nullptr;
   float *topk_val_ = nullptr;
   uint32_t *htopk_ = nullptr;
+  // pinned slots that a snapshot passes through: the gather kernel fills them at ~50 GB/s while the host copies the piece
+  // before.  Pageable copies, two per layer, reach ~4 GB/s.  Snapshots of 0.1 / 1 / 6.3 / 60 MB: 77 / 98 / 560 / 19300 us by
+  // those, 18 / 57 / 300 / 5200 us now
+  static constexpr size_t kSnapSlots = 4, kSnapSlot = 1 << 19;
+  uint8_t *snap_host_ = nullptr;
+  hipEvent_t snap_ev_[kSnapSlots] = {};
   int *hstatus_ = nullptr, *dstatus_ = nullptr;   // attention status word: mapped pinned host memory, its device alias
   void topk_to_host(int M, int *idx, float *val);
   hipGraphExec_t g_state_ = nullptr, g_logits_ = nullptr, g_greedy_ = nullptr;

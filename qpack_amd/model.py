@@ -2,6 +2,7 @@
 (/root/reference/include/qpack/qpack.h:128-171).  Used by the tests and bench.py; C++ callers use include/qpack_hip.h
 directly."""
 import ctypes as C
+import mmap
 
 import numpy as np
 
@@ -14,6 +15,15 @@ def _fptr(a):
 
 def _iptr(a):
     return a.ctypes.data_as(C.POINTER(C.c_int))
+
+
+# a bytes object of a given size, not yet filled, and its address
+_new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.restype, _new_bytes.argtypes = C.py_object, [C.c_void_p, C.c_ssize_t]
+_bytes_address = C.pythonapi.PyBytes_AsString
+_bytes_address.restype, _bytes_address.argtypes = C.c_void_p, [C.py_object]
+_madvise = C.CDLL(None).madvise
+_madvise.restype, _madvise.argtypes = C.c_int, [C.c_void_p, C.c_size_t, C.c_int]
 
 
 class HipLlama:
@@ -129,9 +139,13 @@ class HipLlama:
     def snapshot(self):
         n = C.c_int64(0)
         check(lib().qph_snapshot_size(self._h, C.byref(n)))
-        buf = np.empty(n.value, np.uint8)
-        check(lib().qph_snapshot(self._h, buf.ctypes.data_as(C.c_void_p), n.value))
-        return buf.tobytes()
+        out = _new_bytes(None, n.value)   # filled in place: a copy of a long cache costs as much as reading it back
+        at = _bytes_address(out)
+        if n.value >= 4 << 20:            # huge pages, as numpy asks for: a fault for every 4 KiB takes longer than the copy
+            page = -(-at // 4096) * 4096
+            _madvise(page, at + n.value - page, mmap.MADV_HUGEPAGE)
+        check(lib().qph_snapshot(self._h, at, n.value))
+        return out
 
     def restore(self, s):
         buf = np.frombuffer(s, np.uint8)

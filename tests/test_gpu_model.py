@@ -143,6 +143,24 @@ def test_errors_are_reported(synth):
         qa.HipLlama.load("/nonexistent.qpack")
 
 
+@pytest.mark.parametrize("cfg", ["mini", "mini128"])
+@pytest.mark.parametrize("total", [0, 1, 1 << 19, (1 << 19) + 1, 4 << 19, 9 << 20])
+def test_snapshot_returns_what_restore_took(cfg, total, synth):
+    """snapshots of no position, of one, and of sizes at the edges of the 512 KiB pieces they are read in (one piece, one
+    more row, as many pieces as there are slots, more): byte for byte what restore took"""
+    shape = qa.CONFIGS[cfg]
+    row = 4 * shape.layers * shape.kv_heads * shape.head_dim
+    pos = -(-total // row)
+    body = np.random.default_rng(total).integers(0, 65536, pos * row // 2).astype(np.uint16)
+    snap = np.int32(pos).tobytes() + body.tobytes()
+    print(f"{cfg}: snapshot of {pos} positions, {len(snap)} bytes", flush=True)
+    gpu = qa.HipLlama.load(synth(cfg), max_ctx=pos + 3)
+    gpu.restore(snap)
+    for _ in range(2):
+        assert gpu.snapshot() == snap
+    gpu.close()
+
+
 def split_snapshot(snap, layers, kvd):
     """the reference snapshot layout (model_llama.cpp:55-63): int32 pos, then per layer K rows then V rows (fp16)"""
     pos = int(np.frombuffer(snap[:4], np.int32)[0])
