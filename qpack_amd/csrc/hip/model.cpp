@@ -231,6 +231,11 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
   QPH_CK(hipHostMalloc((void **)&hctl_, kRing * sizeof(Ctl), hipHostMallocDefault));
   QPH_CK(hipHostMalloc((void **)&hout_, 4ull * std::max(V, d), hipHostMallocDefault));
   QPH_CK(hipHostMalloc((void **)&htok_, 4ull * (ctx_ + 1), hipHostMallocDefault));
+  if (vf_ok_) {   // prefill_all's second row buffer, touched here like the snapshot's slots
+    QPH_CK(hipHostMalloc((void **)&vf_host_, 4ull * V, hipHostMallocDefault));
+    memset(vf_host_, 0, 4ull * V);
+    for (hipEvent_t &e : vf_ev_) QPH_CK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
   QPH_CK(hipHostMalloc((void **)&snap_host_, kSnapSlots * kSnapSlot, hipHostMallocDefault));
   memset(snap_host_, 0, kSnapSlots * kSnapSlot);   // its pages' first touch: about a microsecond each, here and not in a first snapshot
   for (hipEvent_t &e : snap_ev_) QPH_CK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -706,10 +711,6 @@ void HipLlama::prefill_all(const int *toks, int n, float *logits) {
 
 void HipLlama::verify_batch(const int *toks, int n, bool fused, float *logits) {
   const int d = cfg_.hidden, ff = cfg_.ffn, V = cfg_.vocab;
-  if (!vf_host_) {
-    QPH_CK(hipHostMalloc((void **)&vf_host_, 4ull * V, hipHostMallocDefault));
-    for (hipEvent_t &e : vf_ev_) QPH_CK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  }
   auto quant = [&](int pro, const float *x, int ldx, const float *w, int cols) {
     PfQuantArgs a{}; a.x = x; a.ldx = ldx; a.norm_w = w; a.eps = cfg_.rms_eps; a.cols = cols;
     a.th = pf_th_; a.tl = pf_tl_; a.ldq = pf_ldq_; a.xb = pf_xb_; a.ldb = pf_ldb_;
