@@ -26,7 +26,7 @@ __device__ __forceinline__ void lds_barrier() {
 
 // ------------------------------------------------------------------ q8, K split over the waves
 // Tile: 16 RT weight rows x 16 NTT tokens per workgroup, 8 waves.  Round r: wave w forms the exact int32 block sums of
-// block 8 r + w for the whole tile on v_mfma_i32_16x16x64_i8 - weights straight from HBM into registers, activations in the order the quantiser leaves for it (PfQuantArgs::tiled: a fragment is
+// block 8 r + w for the whole tile on v_mfma_i32_16x16x64_i8 - weights straight from HBM into registers, activations in the order the quantiser leaves for it (PfQuantArgs::th: a fragment is
 // 1 KiB of consecutive bytes) - T = hi plane, T = 256 T + 128 sum(W), then the lo plane on top (sum(W) from the same fragments against a constant
 // plane), and leaves (float)T in LDS.  After one barrier every thread carries its four rows' fp32 chain over the round's eight blocks in order,
 // acc = fma(bs, (float)isum, acc): rows_q8's order (kernels_x86.cpp:55-71), bit-identical to the tiled products.  The sums
@@ -356,8 +356,9 @@ hipError_t launch_skinny(const GemmArgs &a, int rt, int ntt, int cus, hipStream_
 //   blk = sum over the block's groups of scale * sum, acc = fma(bs[token][block], blk, acc)
 // q1 on the int8 matrix cores, which do twice the columns in the time: a group is a whole block (128 columns, two steps),
 // so the integer work after it is a fourth of q4's.  A bit becomes the byte +-64 (0x40 or 0xc0: a shift, a mask and an
-// or for four); with T = 32 sum(W) + the hi plane, 256 T + the plane lo - 128 = 64 times the group's sum, exact in int32 and as a
-// float (the sum is below 2^22), and 1 / 64 goes into the scale.  64 sum(W) is one more product, with a constant plane.
+// or for four; a set bit, weight +1, is -64); with T = 32 sum(W) + the hi plane, 256 T + the plane lo - 128 = 64 times the
+// group's sum, exact in int32 and as a float (the sum is below 2^22), and -1 / 64 goes into the scale.  64 sum(W) is one more
+// product, with a constant plane.
 // Tile: 16 RT rows x 16 NTT tokens per workgroup; its 8 waves take every eighth block each, add no barrier until the tile's
 // end, and their fp32 partials are summed there in wave order through LDS, 32 tokens at a time.
 // Operands: weights from HBM to registers as stored.  q4: lane l loads the 16 bytes of group l / 16 of row l % 16; a 4 x 4
