@@ -360,7 +360,10 @@ hipError_t launch_skinny(const GemmArgs &a, int rt, int ntt, int cus, hipStream_
 // group's sum, exact in int32 and as a float (the sum is below 2^22), and -1 / 64 goes into the scale.  64 sum(W) is one more
 // product, with a constant plane.
 // Tile: 16 RT rows x 16 NTT tokens per workgroup; its 8 waves take every eighth block each, add no barrier until the tile's
-// end, and their fp32 partials are summed there in wave order through LDS, 32 tokens at a time.
+// end, and their fp32 partials are summed there through LDS, 32 tokens at a time: pairwise, so that the error is below one
+// chain's at every block count above 8 (in rounding variances of one block's size, 9 blocks: chain 45, in wave order 52,
+// pairwise 37; 38: 741, 282, 224).  Up to 8 blocks a wave has one at most and any such sum would round each block once more than
+// the chain acc = fma(bs, blk, acc) does; the waves then leave blk itself and the chain runs at the end.
 // Operands: weights from HBM to registers as stored.  q4: lane l loads the 16 bytes of group l / 16 of row l % 16; a 4 x 4
 // transpose of dwords over the four 16-lane rows (permlane swaps) gives every lane dword l / 16 of each group, and a dword
 // becomes four half pairs with a mask, 0x6400 (1024 + nibble) and one packed subtraction.  q1: dword l / 16 of the block.
@@ -404,7 +407,7 @@ __device__ __forceinline__ v4i q1_bytes16(uint32_t w, int s, uint32_t c) {
   return __builtin_bit_cast(v4i, make_uint4(p[0], p[1], p[2], p[3]));
 }
 
-template <int KIND, int RT, int NTT>
+template <int KIND, int RT, int NTT, bool ORD>
 __global__ __launch_bounds__(kSkWaves * 64) void k_lowbit(GemmArgs a, int nrt, int ntk, int tg, int rg) {
   constexpr bool Q4 = KIND == MK_Q4;
   constexpr int RW = 16 * RT, NT = 16 * NTT, P = RW + 4, SB = Q4 ? 8 : 2;   // SB: scale bytes per row and block
@@ -576,7 +579,7 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_lowbit(GemmArgs a, int nrt, i
 #pragma unroll
         for (int n = 0; n < NTT; n++)
 #pragma unroll
-          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(bs[n], blk[i][n][r], acc[i][n][r]);
+          for (int r = 0; r < 4; r++) acc[i][n][r] = ORD ? blk[i][n][r] : __builtin_fmaf(bs[n], blk[i][n][r], acc[i][n][r]);
     } else {
       v4i F[2][RT], R[RT];
       const v4i ones = (v4i){0x01010101, 0x01010101, 0x01010101, 0x01010101};
@@ -614,7 +617,10 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_lowbit(GemmArgs a, int nrt, i
 #pragma unroll
         for (int i = 0; i < RT; i++)
 #pragma unroll
-          for (int r = 0; r < 4; r++) acc[i][n][r] = __builtin_fmaf(bs[n], w[i][r] * (float)T[i][r], acc[i][n][r]);
+          for (int r = 0; r < 4; r++) {
+            const float blk = w[i][r] * (float)T[i][r];
+            acc[i][n][r] = ORD ? blk : __builtin_fmaf(bs[n], blk, acc[i][n][r]);
+          }
       }
     }
     bj = bj + 1 < nj ? bj + 1 : 0;
@@ -631,11 +637,21 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_lowbit(GemmArgs a, int nrt, i
         for (int i = 0; i < RT; i++)
           *(f4v *)(red + (wave * RT16 + 16 * (n - n0) + lr) * P + 16 * i + 4 * lg) = acc[i][n];
       lds_barrier();
+      auto part = [&](int w, int tok, int row) { return *(const f4v *)(red + (w * RT16 + tok) * P + row); };
       auto sum = [&](int tok, int row) {
-        f4v v = *(const f4v *)(red + tok * P + row);
+        if constexpr (ORD) {
+          f4v v = (f4v){0.f, 0.f, 0.f, 0.f};
+          for (int w = 0; w < nb; w++) {
+            const f4v p = part(w, tok, row);
+            const float bs = bsl[w * NT + 16 * n0 + tok];
 #pragma unroll
-        for (int w = 1; w < kSkWaves; w++) v += *(const f4v *)(red + (w * RT16 + tok) * P + row);
-        return v;
+            for (int r = 0; r < 4; r++) v[r] = __builtin_fmaf(bs, p[r], v[r]);
+          }
+          return v;
+        } else {
+          return ((part(0, tok, row) + part(1, tok, row)) + (part(2, tok, row) + part(3, tok, row))) +
+                 ((part(4, tok, row) + part(5, tok, row)) + (part(6, tok, row) + part(7, tok, row)));
+        }
       };
       const int quads = paired ? RW / 8 : RW / 4, ntoks = NTT - n0 < RN ? 16 * (NTT - n0) : RT16;
       for (int e = tid; e < ntoks * quads; e += kSkWaves * 64) {
@@ -696,16 +712,20 @@ static int lowbit_row_tiles(const GemmArgs &a, int rt) {
   for (int s = 0; s < a.nseg; s++) n += (a.seg[s].rows + rw - 1) / rw;
   return n;
 }
-template <int KIND, int RT, int NTT>
-static hipError_t launch_lowbit_t(const GemmArgs &a, int cus, hipStream_t st) {
+template <int KIND, int RT, int NTT, bool ORD>
+static hipError_t launch_lowbit_o(const GemmArgs &a, int cus, hipStream_t st) {
   const int nrt = lowbit_row_tiles(a, RT), nt16 = (a.ntok + 15) / 16, ntk = (nt16 + NTT - 1) / NTT;
   int sets, tg;
   lowbit_sets(ntk, &sets, &tg);
   const int per = sk_tiles_per_wg(nrt, tg, cus), rg = ((nrt + 7) / 8 + per - 1) / per;
   const size_t lds = lowbit_lds(KIND, RT, NTT, a.cols / kQB);
   if (lds > 160 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_lowbit<KIND, RT, NTT>), dim3((unsigned)(8 * sets * tg * rg)), dim3(kSkWaves * 64), lds, st, a, nrt, ntk, tg, rg);
+  hipLaunchKernelGGL((k_lowbit<KIND, RT, NTT, ORD>), dim3((unsigned)(8 * sets * tg * rg)), dim3(kSkWaves * 64), lds, st, a, nrt, ntk, tg, rg);
   return hipGetLastError();
+}
+template <int KIND, int RT, int NTT>
+static hipError_t launch_lowbit_t(const GemmArgs &a, int cus, hipStream_t st) {
+  return a.cols / kQB <= kSkWaves ? launch_lowbit_o<KIND, RT, NTT, true>(a, cus, st) : launch_lowbit_o<KIND, RT, NTT, false>(a, cus, st);
 }
 // The tile shape for a launch: a start of ~5 us, then per row tile of a workgroup every wave's blocks and ~1 us for each
 // pass of its end (block times with every CU busy, fitted to the shapes above, within 10 % of what they take).  32-row
