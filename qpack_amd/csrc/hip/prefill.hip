@@ -858,7 +858,7 @@ hipError_t launch_pf_rope(const PfRopeArgs &a, int B, hipStream_t st) {
 // ------------------------------------------------------------------ causal attention of a token batch (f16 MFMA)
 // Token t (position P = p0 + t) attends to cache positions [0, P] - the prompt path of model_llama.cpp:95-105.
 // A wave owns one unit = (16-token tile, query head); a workgroup's 8 waves share the kv group and stream its cache in
-// 32-position blocks through LDS (K as stored, V transposed), with an online softmax per token:
+// 64-position blocks through LDS (K as stored, V transposed), with an online softmax per token:
 //   scores  S^T[p][t] = K[p] . q[t] on v_mfma_f32_16x16x32_f16: A = K rows (exact fp16), B = q^T; q is fp32, so it
 //           enters as hi + lo halves (hi = f16(q), lo = f16(q - hi)) - two MFMAs, products exact, fp32 accumulation;
 //           q is pre-scaled by log2(e) / sqrt(hd) (the reference's 1 / sqrt(hd), in base-2 units);
@@ -871,7 +871,10 @@ hipError_t launch_pf_rope(const PfRopeArgs &a, int B, hipStream_t st) {
 //           kernel's order (the reference-order mode has its own kernel, k_ex_pf_attn).
 constexpr int kPfKB = 64;      // cache positions per block (two 32-deep value steps)
 constexpr int kPfAttnWaves = 8;   // units (16-token tile, query head) per workgroup, one per wave: they share the K / V
-template <int HD>
+// SPLIT (a share of the cache per workgroup, pf_attn_splits) is a template parameter: decided at run time, the share's
+// bounds and the partials' store in the same code slowed the unsplit kernel by 9 % (700 / 1024 / 2048 tokens behind 16384
+// positions, 32 heads in 8 groups: 753 / 812 / 1637 us against 673 / 743 / 1502)
+template <int HD, bool SPLIT>
 __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
   typedef float f4 __attribute__((ext_vector_type(4)));
@@ -895,7 +898,7 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
   const int L = blockIdx.y * gridDim.x + blockIdx.x;
   // with splits: the workgroups of one (group, share of its cache) on one XCD, whose L2 then reads that share once
   int bx = gridDim.x - 1 - L / gridDim.y, g = L % gridDim.y, z = 0;
-  if (a.nsplit > 1) {
+  if constexpr (SPLIT) {
     const int k = L >> 3, pair = k / gridDim.x * 8 + (L & 7);
     if (pair >= a.nkv * a.nsplit) return;
     bx = gridDim.x - 1 - k % gridDim.x; g = pair % a.nkv; z = pair / a.nkv;
@@ -913,7 +916,7 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
   const int ulast = min(bx * kPfAttnWaves + kPfAttnWaves - 1, nunits - 1);
   const int wg_last = a.p0 + min((ulast / rep) * 16 + 15, a.ntok - 1);
   // its cache blocks; with splits share z of them
-  const int nkb_all = wg_last / kPfKB + 1, kb0 = nkb_all * z / a.nsplit, nkb = nkb_all * (z + 1) / a.nsplit;
+  const int nkb_all = wg_last / kPfKB + 1, kb0 = SPLIT ? nkb_all * z / a.nsplit : 0, nkb = SPLIT ? nkb_all * (z + 1) / a.nsplit : nkb_all;
 
   // q^T fragments: lane holds q[t][32 s + 8 lg + 0..7] as hi / lo halves, pre-scaled by log2(e) / sqrt(hd) so the
   // scores come out in base-2 units for the hardware exp2 (v_exp_f32)
@@ -1069,7 +1072,7 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
     }
   }
   if (!tok_ok) return;   // a token's four lanes (lr, l ^ 16, l ^ 32, l ^ 48) leave together
-  if (a.nsplit > 1) {   // unnormalised output and (max, sum) for k_pf_attn_merge (max -inf: no position in this share)
+  if constexpr (SPLIT) {   // unnormalised output and (max, sum) for k_pf_attn_merge (max -inf: no position in this share)
     const size_t th = ((size_t)z * a.ntok + t) * a.nh + head;
     if (lg == 0) *(float2 *)(a.part + (size_t)a.nsplit * a.ntok * a.nh * HD + 2 * th) = make_float2(m, l);
 #pragma unroll
@@ -1192,8 +1195,10 @@ hipError_t launch_pf_attn(const PfAttnArgs &a0, hipStream_t st) {
   if (most > 1) a.nsplit = pf_attn_splits((int)grid.x, a.nkv, blocks, gemm_cus(), most);
   if (const char *e = getenv("QPH_PF_SPLIT")) a.nsplit = std::max(1, std::min(most, atoi(e)));   // test hook
   if (a.nsplit > 1) grid.y = (a.nkv * a.nsplit + 7) / 8 * 8;
-  if (a.hd == 128) hipLaunchKernelGGL(k_pf_attn<128>, grid, dim3(kPfAttnWaves * 64), 0, st, a);
-  else hipLaunchKernelGGL(k_pf_attn<64>, grid, dim3(kPfAttnWaves * 64), 0, st, a);
+#define QPH_PFA(HD, SPLIT) hipLaunchKernelGGL((k_pf_attn<HD, SPLIT>), grid, dim3(kPfAttnWaves * 64), 0, st, a)
+  if (a.hd == 128) { if (a.nsplit > 1) QPH_PFA(128, true); else QPH_PFA(128, false); }
+  else { if (a.nsplit > 1) QPH_PFA(64, true); else QPH_PFA(64, false); }
+#undef QPH_PFA
   if (a.nsplit > 1) {
     const dim3 mg((a.ntok * a.nh + 3) / 4);
     if (a.hd == 128) hipLaunchKernelGGL(k_pf_attn_merge<128>, mg, dim3(256), 0, st, a);
