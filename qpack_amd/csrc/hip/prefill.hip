@@ -727,17 +727,20 @@ static int gemm_row_tiles(const GemmArgs &a, bool big) {
   for (int s = 0; s < a.nseg && s < kGemmMaxSeg; s++) t += (a.seg[s].rows + rt - 1) / rt;
   return t;
 }
-// The few-token kernel against the 128-row tiles: a round of those takes ~1.35 us per 128-column block whatever part of
-// it is filled (4096 x 14336 at 16 .. 128 tokens 126 .. 156 us, 14336 x 4096 pairs 48 .. 55, 6144 x 4096 39 .. 42).  The
-// lines that follow from it: 6144 x 4096 and 4096 x 14336 from 512 tokens to the tiles (512: 69 against 46 us, 149 against
-// 156), 4096 x 4096 from 384, gate / up pairs of 14336 x 4096 from 48 (40: 46 against 51 us; 77: 69 against 53)
+// The few-token kernel against the 128-row tiles: those take ~5 us, then a round ~3 us and ~1.18 us per 128-column block
+// whatever part of it is filled (896 x 896 16 us, 4096 x 4096 44 .. 53, 896 x 4864 51, 4096 x 14336 132 .. 159).  The lines
+// that follow, at shapes of 0.5B and 8B models: 896 x 4864 from 1025 tokens to the tiles (1024: 36 against 51 us; 1152: 57
+// against 51), 4096 x 14336 and 4096 x 4096 from 385 (384: 125 and 41 against 157 and 52; 400: 137 and 46 against 133 and
+// 45), 6144 x 4096 from 257 (256: 36 against 51, 288: 46 against 44), gate / up pairs of 14336 x 4096 from 48.  Of 31 token
+// counts from 96 to 2048 at each of these and 1152 x 896, 896 x 896 and pairs of 4864 x 896, the pick is within 9 % of the
+// faster kernel
 bool gemm_wants_tiles(const GemmArgs &a) {
   if (a.kind != MK_Q8 || a.ntok <= 0 || a.cols % kQB) return false;
   if (const int f = gemm_forced()) return f == 3;
   const bool big = gemm_uses_32x32(a);
   const long wgs = (long)gemm_row_tiles(a, big) * ((a.ntok + kGN - 1) / kGN);
   int rt, ntt;
-  return skinny_cost(a, gemm_cus(), &rt, &ntt) < 5 + gemm_rounds(wgs) * (big ? kG2Cost : 1.0) * 1.35 * (a.cols / kQB);
+  return skinny_cost(a, gemm_cus(), &rt, &ntt) < 5 + gemm_rounds(wgs) * (big ? kG2Cost : 1.0) * (3 + 1.18 * (a.cols / kQB));
 }
 bool gemm_uses_32x32(const GemmArgs &a) {
   return a.kind == MK_Q8 && a.xbt && a.ntok > 0 && gemm_use_32x32(gemm_row_tiles(a, true), (a.ntok + kG2N - 1) / kG2N);

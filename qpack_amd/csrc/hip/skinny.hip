@@ -318,22 +318,28 @@ static hipError_t launch_skinny_t(const GemmArgs &a, int nrt, int cus, hipStream
   return hipGetLastError();
 }
 // The tile shape and the time it is expected to take: a start of ~5 us, then per row tile of a workgroup its rounds and
-// ~0.8 us for its end (round times from the shapes above and 14336 x 4096 pairs, with every CU busy)
+// ~0.8 us for its end (round times from the shapes above and 14336 x 4096 pairs, with every CU busy).  Every XCD reads the
+// tokens' planes once per row tile: beyond its 4 MiB of L2 they come from the shared cache, all XCDs together at ~7 TB/s,
+// and a row tile takes no less than that (896 x 4864 at 1152 / 1536 / 2048 tokens, expected by the rounds alone 54 / 54 / 60
+// us: 57 / 72 / 97, with this 59 / 76 / 99; 4096 x 14336 at 2048 600: 1057, with this 1089)
 double skinny_cost(const GemmArgs &a, int cus, int *rt, int *ntt) {
   static const double round_us[2][4] = {{1.05, 1.3, 1.9, 1.9}, {1.5, 1.9, 2.3, 2.6}};
   const int rounds = (a.cols / kQB + kSkWaves - 1) / kSkWaves, nt16 = (a.ntok + 15) / 16;
+  const double planes = 32.0 * nt16 * a.cols, planes_us = planes > 4e6 ? planes * 8 / 7e6 : 0;
   double best = 1e30;
   for (int r = a.w2 ? 2 : 1; r <= 2; r++)
     for (int n = 1; n <= 4; n++) {
       const int ntk = (nt16 + n - 1) / n, per = sk_tiles_per_wg(sk_row_tiles(a, r), ntk, cus);
       const int waves = (8 * ntk + cus - 1) / cus;   // more token tiles than CUs / 8: several workgroups to a CU
-      const double c = 5 + waves * per * (rounds * round_us[r - 1][n - 1] + 0.8);
+      const double c = 5 + per * (std::max(waves * rounds * round_us[r - 1][n - 1], planes_us) + waves * 0.8);
       if (c < best) { best = c; *rt = r; *ntt = n; }
     }
   return best;
 }
 hipError_t launch_skinny(const GemmArgs &a, int rt, int ntt, int cus, hipStream_t st) {
-  if (a.kind != MK_Q8 || a.ldb % 8 || a.ldb < round_up(a.cols / kQB, 8) || (a.w2 && rt != 2)) return hipErrorInvalidValue;
+  if (a.kind != MK_Q8 || a.ldb % 8 || a.ldb < round_up(a.cols / kQB, 8) || (a.w2 && rt != 2) ||
+      (size_t)round_up(a.ntok, 16) * a.ldq >> 32)   // the kernel's offsets into a plane are 32 bits
+    return hipErrorInvalidValue;
   const int nrt = sk_row_tiles(a, rt);
   if (a.deal.waves > 0 || a.group_blocks > 0) {   // the decode step's orders: one tile of at most 16 tokens
     if (a.ntok > 16 || a.nseg > 1 || (a.deal.waves > 0 && (a.group_blocks > 0 || a.deal.ns < 1)) || (a.group_blocks > 0 && a.w2))
