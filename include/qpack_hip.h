@@ -132,6 +132,9 @@ int qph_time_greedy(qph_model *m, int token, int n, float *ms);
  * which: 0 = fused RMSNorm + gate/up + SwiGLU matvec, 1 = down matvec, 2 = fused RMSNorm + qkv matvec, 3 = wo matvec,
  * 4 = output head matvec + argmax partials, 5 = attention at the current position. */
 int qph_time_kernel(qph_model *m, int which, int iters, float *ms, double *bytes);
+/* The batches that prefill_all has run on this model so far (q8 models in the default order: runs of 2 to 16 tokens; the
+ * tokens of other models and single ones take decode steps, with the same bits). */
+int qph_verify_batches(const qph_model *m, int64_t *n);
 /* A plain device-to-device copy of `bytes` (a multiple of 16) through the kernel k_copy, `iters` times on a stream of
  * its own, with the buffers allocated and freed inside; *ms = mean HIP-event duration.  Calibrates hardware byte
  * counters (a profiler's FETCH_SIZE / WRITE_SIZE of k_copy should read `bytes` each). */

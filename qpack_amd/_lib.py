@@ -72,6 +72,7 @@ SIGNATURES = {
     "qph_set_order": (_I, [_P, _I]),
     "qph_time_greedy": (_I, [_P, _I, _I, _FP]),
     "qph_time_kernel": (_I, [_P, _I, _I, _FP, C.POINTER(C.c_double)]),
+    "qph_verify_batches": (_I, [_P, C.POINTER(C.c_int64)]),
     "qph_time_copy": (_I, [C.c_int64, _I, _FP]),
     "qph_kernel_matvec": (_I, [_I, _P, _P, _I, _I, _FP, _FP, C.POINTER(C.c_int32), C.POINTER(C.c_int16), _FP]),
     "qph_kernel_matmul": (_I, [_I, _P, _P, _I, _I, _FP, _I, _FP]),

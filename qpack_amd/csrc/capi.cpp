@@ -134,6 +134,9 @@ int qph_greedy_run(qph_model *m, int token, int n, int *out, int *produced) {
     if (produced) *produced = r;
   });
 }
+int qph_verify_batches(const qph_model *m, int64_t *n) {
+  QPH_API_TRY({ need(m, "model"); need(n, "n"); *n = m->m->verify_batches(); });
+}
 int qph_prefill_all(qph_model *m, const int *tokens, int n, float *logits) {
   QPH_API_TRY({ need(m, "model"); need(tokens, "tokens"); need(logits, "logits"); m->m->prefill_all(tokens, n, logits); });
 }

@@ -196,7 +196,11 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
     pf_ldq_ = (int)(wide + 15) / 16 * 16;
     pf_x_ = (float *)dalloc(4 * B * d); pf_q_ = (float *)dalloc(4 * B * qd_); pf_att_ = (float *)dalloc(4 * B * qd_);
     pf_k_ = (float *)dalloc(4 * B * kvd_); pf_v_ = (float *)dalloc(4 * B * kvd_);
-    pf_g_ = (float *)dalloc(4 * B * ff);
+    // batched prefill_all: q8 throughout, and the fused attention adds its parts itself
+    vf_ok_ = !half_mats && head_.kind == MK_Q8 && (awo_max_ <= 0 || awo_rows_ || awo_sum_);
+    const size_t vn = vf_ok_ ? std::min<size_t>(kVerify, B) : 0;   // tokens of a batch
+    // its attention partials and logits are left in the gate / up output's buffer, whatever the context window
+    pf_g_ = (float *)dalloc(4 * std::max(B * ff, vn * std::max<size_t>(V, (size_t)nh * max_chunks_ * (hd + 2))));
     pf_xh_ = (int8_t *)dalloc(B * pf_ldq_); pf_xl_ = (int8_t *)dalloc(B * pf_ldq_);
     const size_t B16 = (B + 15) / 16 * 16;
     if (q8_mats) {
@@ -211,11 +215,7 @@ HipLlama::HipLlama(const qph_config &cfg, const qph_tensor *tensors, int n, int 
     pf_xbt2_ = (float *)dalloc(4ull * pf_ldbt_ * (pf_ldq_ / 128 + 1));
     if (half_mats) pf_fp_ = (uint16_t *)dalloc(4 * B16 * wide);
     pf_tok_ = (int *)dalloc(4 * B);
-    // batched prefill_all: q8 throughout, the scratch (the gate / up output's buffer: attention partials, logits) fits, and
-    // the fused attention adds its parts itself
-    vf_ok_ = !half_mats && head_.kind == MK_Q8 && (awo_max_ <= 0 || awo_rows_ || awo_sum_) && B >= (size_t)kVerify &&
-             B * ff >= (size_t)kVerify * std::max<size_t>(V, (size_t)nh * max_chunks_ * (hd + 2));
-    if (vf_ok_) vf_q16_ = (uint16_t *)dalloc(4ull * kVerify * qd_);
+    if (vf_ok_) vf_q16_ = (uint16_t *)dalloc(4 * vn * qd_);
   }
   // RoPE tables in the reference's precision: inv_i = 1 / theta^(2i/hd) and angle pos * inv_i in double, cos / sin
   // rounded to float (model_llama.cpp:39, :173-175)
@@ -695,14 +695,16 @@ int HipLlama::greedy_run(int tok, int n, int *out) {
 
 // Model::prefill_all: every token's logits equal its decode step's bit for bit (the reference's ExactBatches contract).
 // q8 models in the default order: batches of up to kVerify tokens through products that read the weights once and sum in
-// the decode kernels' orders; a batch stays on one side of the fused attention's limit, whose order differs.
+// the decode kernels' orders; a batch stays on one side of the fused attention's limit, whose order differs.  Two tokens
+// already take less than two steps (behind 600 positions 1103 against 1184 us on eight layers of the 8B shape, 1431 against
+// 1578 on the 0.5B one), a third one costs 30 us more instead of 590 and 780.
 void HipLlama::prefill_all(const int *toks, int n, float *logits) {
   if (pos_ + n > ctx_) throw std::runtime_error("context window full (" + std::to_string(ctx_) + " tokens)");
   const bool batched = vf_ok_ && !order_ && !getenv("QPH_VERIFY_STEPS");   // test hook: decode steps
   for (int i = 0; i < n;) {
     int m = 0;   // tokens of this batch: valid ids, one regime
     const bool fused = pos_ + 1 <= awo_max_;
-    while (batched && m < kVerify && i + m < n && toks[i + m] >= 0 && toks[i + m] < cfg_.vocab &&
+    while (batched && m < std::min(kVerify, pf_cap_) && i + m < n && toks[i + m] >= 0 && toks[i + m] < cfg_.vocab &&
            (pos_ + m + 1 <= awo_max_) == fused) m++;
     if (m > 1) { verify_batch(toks + i, m, fused, logits + (size_t)i * cfg_.vocab); i += m; }
     else { step(toks[i], 1, logits + (size_t)i * cfg_.vocab); i++; }
@@ -722,6 +724,7 @@ void HipLlama::verify_batch(const int *toks, int n, bool fused, float *logits) {
     return a;
   };
   const int p0 = pos_;
+  vf_batches_++;
   write_ctl(toks[0], p0);
   QPH_CK(hipMemcpyAsync(pf_tok_, toks, 4ull * n, hipMemcpyHostToDevice, st_));
   QPH_CK(launch_pf_embed(embed_, pf_tok_, n, pf_x_, d, st_));

@@ -31,6 +31,7 @@ class HipLlama {
   void prefill(const int *toks, int n, int want, float *out);
   int greedy_run(int tok, int n, int *out);
   void prefill_all(const int *toks, int n, float *logits);
+  int64_t verify_batches() const { return vf_batches_; }
   // step / prefill whose logits stay on the device and come back as their M largest (index, value) pairs, in the
   // sampler's order (1 <= M <= min(kTopkMax, vocab))
   void step_topk(int tok, int M, int *idx, float *val);
@@ -162,6 +163,7 @@ class HipLlama {
   // prefill_all in batches of up to kVerify tokens whose every logit equals its decode step's bit for bit (q8 models)
   static constexpr int kVerify = 16;
   bool vf_ok_ = false;
+  int64_t vf_batches_ = 0;       // batches run so far
   uint16_t *vf_q16_ = nullptr;   // [kVerify][2 qd_]
   float *vf_host_ = nullptr;     // pinned: the second row buffer of the logits' way to the host
   hipEvent_t vf_ev_[2] = {};

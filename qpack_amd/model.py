@@ -160,6 +160,12 @@ class HipLlama:
         return {"planes": st.planes, "coded_bytes": st.coded_bytes, "raw_bytes": st.raw_bytes, "upload_ms": st.upload_ms,
                 "decode_ms": st.decode_ms, "total_ms": st.total_ms, "rounds": st.rounds}
 
+    def verify_batches(self):
+        """the batches that prefill_all has run on this model so far"""
+        n = C.c_int64(0)
+        check(lib().qph_verify_batches(self._h, C.byref(n)))
+        return n.value
+
     def time_greedy(self, token, n):
         ms = C.c_float(0)
         check(lib().qph_time_greedy(self._h, int(token), int(n), C.byref(ms)))

@@ -363,7 +363,9 @@ def test_prefill_all_batches_equal_decode_steps(cfg, T, awo, synth, monkeypatch)
     """prefill_all of a q8 model in batches: the logits of every token and the cache rows equal the decode steps' bit for
     bit (QPH_VERIFY_STEPS) - behind short contexts (the fused attention + wo kernels' orders), across the fused limit
     (640 positions, 100 forced, 256 for mini_r7) in one call, at one split, under 16 splits and at 16 and more (960: the
-    first context that merges in its own launch is inside the call), 1, 2, 16 and 37 tokens (batches of 16 and a rest)"""
+    first context that merges in its own launch is inside the call), 1, 2, 16 and 37 tokens (batches of 16 and a rest).  The
+    c1 window of 300 holds fewer gate / up outputs than a batch's logits.  A call of two tokens or more has to run batches,
+    or it compares steps with steps"""
     if awo is not None:
         monkeypatch.setenv("QPH_AWO_MAX", awo)
     path = synth(cfg)
@@ -385,8 +387,11 @@ def test_prefill_all_batches_equal_decode_steps(cfg, T, awo, synth, monkeypatch)
                 monkeypatch.delenv("QPH_VERIFY_STEPS")
             print(f"{cfg}: prefill_all of {n} behind {T}, {'steps' if steps else 'batches'}", flush=True)
             assert gpu.rewind(T)
+            before = gpu.verify_batches()
             out.append((gpu.prefill_all(toks), gpu.snapshot()))
             assert gpu.pos() == T + n
+            ran = gpu.verify_batches() - before
+            assert ran == 0 if steps or n == 1 else -(-n // 16) <= ran <= -(-n // 16) + 1
         for i in range(n):
             np.testing.assert_array_equal(out[0][0][i], out[1][0][i], err_msg=f"token {i} at position {T + i}")
         assert out[0][1] == out[1][1], "cache rows differ"
@@ -396,6 +401,25 @@ def test_prefill_all_batches_equal_decode_steps(cfg, T, awo, synth, monkeypatch)
     with pytest.raises(qa.QphError, match="out of range"):
         gpu.prefill_all(bad)
     assert gpu.pos() == T + 3
+    gpu.close()
+
+
+@pytest.mark.parametrize("cfg,ctx,chunk", [("mini", 9, None), ("mini128", 21, None), ("mini128", 40, "5")])
+def test_prefill_all_small_windows(cfg, ctx, chunk, synth, monkeypatch):
+    """prefill_all that fills context windows of fewer tokens than a batch holds, or little more, and with a prompt chunk of
+    fewer (QPH_PF_CHUNK: the buffers then hold 5): batches of what fits, the bits of the decode steps"""
+    if chunk:
+        monkeypatch.setenv("QPH_PF_CHUNK", chunk)
+    shape = qa.CONFIGS[cfg]
+    toks = np.random.default_rng(ctx).integers(0, shape.vocab, ctx).astype(np.int32)
+    gpu = qa.HipLlama.load(synth(cfg), max_ctx=ctx)
+    print(f"{cfg}: prefill_all of {ctx} tokens, chunk {chunk}", flush=True)
+    got = gpu.prefill_all(toks), gpu.snapshot()
+    assert gpu.verify_batches() == -(-ctx // min(16, ctx, int(chunk or 16)))
+    monkeypatch.setenv("QPH_VERIFY_STEPS", "1")
+    gpu.reset()
+    np.testing.assert_array_equal(got[0], gpu.prefill_all(toks))
+    assert got[1] == gpu.snapshot()
     gpu.close()
 
 
