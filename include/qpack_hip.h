@@ -149,9 +149,10 @@ int qph_time_copy(int64_t bytes, int iters, float *ms);
 int qph_kernel_matvec(int kind, const void *q, const void *scale, int rows, int cols, const float *x, float *y,
                       int32_t *sums, int16_t *xq, float *bs);
 /* Runs the product's batched prefill kernels on one matrix (host buffers; q and scale as in qph_kernel_matvec): each
- * row of X[B, cols] quantised as the decode step quantises it, then Y[B, rows] = X W^T on the int8 matrix cores
+ * row of X[B, cols] quantised as the decode step quantises it, then Y[B, rows] = X W^T on the matrix cores
  * (matmul / mm_q8 / mm_q4, kernels.cpp:97-143, kernels_x86.cpp:287-371).  q8 rows use rows_q8's float epilogue per
- * token, so every Y row equals qph_kernel_matvec on that x; q4 rows have exact int32 group sums and their own fp32 order. */
+ * token, so every Y row equals qph_kernel_matvec on that x; q4 and q1 rows have exact group sums (as f16 products whose
+ * partial sums stay below 2^24, and in int32) and fp32 orders of their own. */
 int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int cols, const float *X, int B, float *Y);
 
 /* The reference-order products of qph_set_order(1) on one matrix: every vector of the first B - B % 4 in the lane

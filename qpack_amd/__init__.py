@@ -3,7 +3,7 @@
   HipLlama.load(path)   - a QPACK1/QPACK2 file on the GPU (the qp::Model surface: step / prefill / greedy_run / ...)
   write_synthetic(...)  - seeded random-init QPACK2 models of the benchmark shapes (C1-C5)
   kernel_matvec(...)    - the product's matvec kernel on one matrix, with its exact int32 accumulators (parity hook)
-  kernel_matmul(...)    - the product's batched prefill kernels on one q8 / q4 matrix (parity hook)
+  kernel_matmul(...)    - the product's batched prefill kernels on one q8 / q4 / q1 matrix (parity hook)
   kernel_topk(...)      - the device top-M selection of step_topk on one vector (parity hook)
 """
 from ._lib import LIB_PATH, QPH_F32, QPH_Q1, QPH_Q4, QPH_Q8, QphError, device_count, lib

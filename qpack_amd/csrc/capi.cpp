@@ -264,10 +264,10 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
   QPH_API_TRY({
     need(q, "q"); need(scale, "scale"); need(X, "X"); need(Y, "Y");
     if (rows <= 0 || B <= 0 || cols <= 0 || cols % 128) throw std::invalid_argument("matmul: rows, B > 0 and cols a positive multiple of 128 required");
-    if (kind != QPH_Q8 && kind != QPH_Q4) throw std::invalid_argument("matmul: kind must be QPH_Q8 or QPH_Q4");
-    const int nb = cols / 128, ldb = (nb + 7) / 8 * 8, G = cols / 32;
-    const size_t qb = kind == QPH_Q8 ? (size_t)rows * cols : (size_t)rows * cols / 2;
-    const size_t sb = kind == QPH_Q8 ? 4ull * rows : 2ull * rows * G;
+    if (kind != QPH_Q8 && kind != QPH_Q4 && kind != QPH_Q1) throw std::invalid_argument("matmul: kind must be QPH_Q8, QPH_Q4 or QPH_Q1");
+    const int nb = cols / 128, ldb = (nb + 7) / 8 * 8, G = cols / 32, mk = kind == QPH_Q8 ? qph::MK_Q8 : kind == QPH_Q4 ? qph::MK_Q4 : qph::MK_Q1;
+    const size_t qb = kind == QPH_Q8 ? (size_t)rows * cols : kind == QPH_Q4 ? (size_t)rows * cols / 2 : (size_t)rows * cols / 8;
+    const size_t sb = kind == QPH_Q8 ? 4ull * rows : kind == QPH_Q4 ? 2ull * rows * G : 2ull * rows * nb;
     std::vector<void *> bufs;
     auto alloc = [&](size_t n) { void *p = nullptr; hck(hipMalloc(&p, n), "hipMalloc"); bufs.push_back(p); return p; };
     try {
@@ -279,7 +279,7 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
       hck(hipMemcpy(dq, q, qb, hipMemcpyHostToDevice), "upload q");
       hck(hipMemcpy(ds, scale, sb, hipMemcpyHostToDevice), "upload scale");
       hck(hipMemcpy(dx, X, 4ull * B * cols, hipMemcpyHostToDevice), "upload X");
-      qph::GemmArgs ga{}; ga.kind = kind == QPH_Q8 ? qph::MK_Q8 : qph::MK_Q4; ga.w = (const int8_t *)dq; ga.scale = (const float *)ds;
+      qph::GemmArgs ga{}; ga.kind = mk; ga.w = (const int8_t *)dq; ga.scale = (const float *)ds;
       ga.rows = rows; ga.cols = cols; ga.xh = dxh; ga.xl = dxl; ga.xb = dxb; ga.ntok = B; ga.ldq = cols; ga.ldb = ldb;
       ga.y = dy; ga.ldy = rows; ga.xbt = dxbt; ga.ldbt = ldbt;
       qph::PfQuantArgs qa{}; qa.x = dx; qa.ldx = cols; qa.cols = cols; qa.xh = dxh; qa.xl = dxl; qa.ldq = cols; qa.xb = dxb; qa.ldb = ldb;
@@ -289,9 +289,9 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
         qa.th = (int8_t *)alloc(tb); qa.tl = (int8_t *)alloc(tb); qa.xh = qa.xl = nullptr;
         ga.th = qa.th; ga.tl = qa.tl;
       }
-      if (kind == QPH_Q4) {
-        qa.fp = (uint16_t *)alloc((size_t)(B + 15) / 16 * 16 * cols * 4);
-        qa.fkind = qph::MK_Q4; ga.fp = qa.fp;
+      if (kind != QPH_Q8) {
+        qa.fp = (uint16_t *)alloc((size_t)(B + 15) / 16 * 16 * cols * (kind == QPH_Q4 ? 4 : 2));
+        qa.fkind = mk; ga.fp = qa.fp;
       }
       hck(qph::launch_pf_quant(qph::PRO_QUANT, qa, B, nullptr), "launch quant");
       if (kind == QPH_Q8) {
@@ -300,7 +300,7 @@ int qph_kernel_matmul(int kind, const void *q, const void *scale, int rows, int 
         ga.wsum = dws;
       } else {
         uint16_t *dst = (uint16_t *)alloc(sb);
-        hck(qph::launch_scale_blocks(qph::MK_Q4, (const uint16_t *)ds, rows, cols, dst, nullptr), "launch scale blocks");
+        hck(qph::launch_scale_blocks(mk, (const uint16_t *)ds, rows, cols, dst, nullptr), "launch scale blocks");
         ga.st = dst;
       }
       hck(qph::launch_gemm(ga, nullptr), "launch gemm");

@@ -204,8 +204,8 @@ def kernel_matvec(kind, q, scale, x):
 
 def kernel_matmul(q, scale, X, kind=None, order=0):
     """the product's batched prefill kernels on one matrix: Y[B, rows] = X[B, cols] W^T (qph_kernel_matmul); q8 (int8
-    q, f32 scale) or q4 (packed u8 q, fp16-bits scale per 32 columns); order=1: the reference-order products
-    (qph_kernel_matmul_ref), which also take kind=QPH_Q1 (sign bits [rows][cols / 8], fp16-bits scale per 128 columns)"""
+    q, f32 scale), q4 (packed u8 q, fp16-bits scale per 32 columns) or, with kind=QPH_Q1, q1 (sign bits [rows][cols / 8],
+    fp16-bits scale per 128 columns); order=1: the reference-order products (qph_kernel_matmul_ref)"""
     from ._lib import QPH_Q1, QPH_Q4, QPH_Q8
     if kind is None:
         kind = QPH_Q8 if q.dtype == np.int8 else QPH_Q4

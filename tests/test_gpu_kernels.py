@@ -130,7 +130,7 @@ def test_matmul_q8_few_tokens(rows, cols, B, tile, monkeypatch):
 @pytest.mark.parametrize("rows,cols,B", [(1000, 4096, 200), (257, 896, 129), (300, 18944, 17), (9, 128, 1), (3584, 3584, 64),
                                          (130, 512, 1024)])
 def test_matmul_q4(rows, cols, B):
-    """batched prefill product on q4 rows (int8 MFMA over unpacked nibbles, exact int32 group sums): every token's row
+    """batched prefill product on q4 rows (f16 MFMA over unpacked nibbles, exact group sums): every token's row
     against rows_q4 on that token's quantised activation, within 2e-6 of the summed term magnitudes (its own fp32
     order); ragged row / token counts exercise the tile edges"""
     rng = np.random.default_rng(rows * 17 + cols + B)
@@ -224,6 +224,46 @@ def test_matmul_q4_no_less_exact_than_one_chain(cols, B, tile, monkeypatch):
     if off:
         rms, chain = np.sqrt(np.mean(np.square(off))), np.sqrt(np.mean(np.square(off_chain)))
         assert rms < chain, (rms, chain)
+
+
+@pytest.mark.parametrize("rows,cols,B", [(7, 128, 1), (31, 1024, 16), (33, 1152, 17), (65, 896, 33), (4113, 2048, 50), (300, 14336, 77),
+                                         (130, 4096, 50), (48, 4864, 129), (2100, 512, 700)])
+@pytest.mark.parametrize("tile", ["", "21", "22", "41", "42", "44"])
+def test_matmul_q1_exact_group_sums(rows, cols, B, tile, monkeypatch):
+    """the q1 product on the int8 matrix cores, the launcher's tile and each one forced: row and token counts around the tile
+    edges, 1, 4, 7, 8, 9, 16, 32, 38 and 112 blocks (waves without a block, with one, with two and more, some with one fewer),
+    several row tiles to a workgroup (4113 and 2100 rows).  A group's sum is exact in int32 and as a float, so up to eight
+    blocks the result is the chain acc = fma(bs, scale * sum, acc) bit for bit.  Extreme inputs: weights all +1 and all -1
+    against activations all at the quantiser's limits (sums of +-128 x 32767), alternating signs among them"""
+    if tile:
+        monkeypatch.setenv("QPH_SKINNY", tile)
+    rng = np.random.default_rng(rows * 31 + cols + B)
+    nb = cols // 128
+    q = rng.integers(0, 256, (rows, cols // 8)).astype(np.uint8)
+    q[0] = 0x00; q[1] = 0xff; q[2] = 0x55
+    s = (rng.random((rows, nb)) * 0.01 + 1e-4).astype(np.float16).view(np.uint16)
+    X = rng.normal(0, 1, (B, cols)).astype(np.float32)
+    X[0] = 3.5                                      # every activation 32767
+    if B > 1:
+        X[1] = -3.5; X[B // 2] = 0
+        X[B - 1] = np.where(np.arange(cols) % 2 == 0, 2.0, -2.0)
+    print(f"q1 product tile {tile or 'auto'} rows={rows} cols={cols} B={B}", flush=True)
+    Y = qa.kernel_matmul(q, s, X, kind=qa.QPH_Q1)
+    sign = np.unpackbits(q, axis=1, bitorder="little").astype(np.int32) * 2 - 1
+    w = s.view(np.float16).astype(np.float32)
+    for b in sorted({0, min(1, B - 1), B - 1, *range(0, B, max(1, B // 12))}):
+        xq, bs = O.quant_act(X[b])
+        gs = (sign.reshape(rows, nb, 128) * xq.astype(np.int32).reshape(1, nb, 128)).sum(2)
+        if nb <= 8:
+            acc = np.zeros(rows, np.float32)
+            for k in range(nb):
+                acc = fma32(bs[k], w[:, k] * gs[:, k].astype(np.float32), acc)
+            np.testing.assert_array_equal(Y[b], acc, err_msg=f"token {b}")
+            continue
+        terms = w.astype(np.float64) * bs.astype(np.float64)[None, :] * gs
+        # fp32: scale * sum rounded once, a chain of ceil(blocks / 8), three additions, 2^-24 each
+        tol = (4 + -(-nb // 8)) * 2.0 ** -24 * np.abs(terms).sum(1)
+        assert np.all(np.abs(Y[b] - terms.sum(1)) <= tol + 1e-30), (b, float(np.max(np.abs(Y[b] - terms.sum(1)) / (tol + 1e-30))))
 
 
 @pytest.mark.parametrize("kind", ["q8", "q4"])
