@@ -311,6 +311,71 @@ def test_batched_prefill_q1(cfg, tile, n, synth, monkeypatch):
     gpu.close(); orc.close()
 
 
+def with_kinds(path, kinds, max_ctx):
+    """the model of `path` with some matrices replaced by random ones of another kind ({tensor suffix: "q4" / "q1" / "q8"}),
+    through qph_create"""
+    import ctypes as C
+
+    from qpack_amd._lib import Config, Tensor, check, lib
+    f = O.QpackFile(path)
+    code = {O.OR_F32: qa.QPH_F32, O.OR_Q8: qa.QPH_Q8, O.OR_Q4: qa.QPH_Q4, O.OR_Q1: qa.QPH_Q1}
+    rng = np.random.default_rng(9)
+    keep, ts = [], []
+    for name in f.tensors:
+        kind, q, s, rows, cols = f.tensor(name)
+        kind, want = code[kind], kinds.get(name.split(".")[-1])
+        if want == "q8":
+            kind, q, s = qa.QPH_Q8, rng.integers(-127, 128, (rows, cols)).astype(np.int8), np.full(rows, 0.0005, np.float32)
+        elif want == "q4":
+            kind, q = qa.QPH_Q4, rng.integers(0, 256, (rows, cols // 2)).astype(np.uint8)
+            s = np.full((rows, cols // 32), 0.004, np.float16)
+        elif want == "q1":
+            kind, q = qa.QPH_Q1, rng.integers(0, 256, (rows, cols // 8)).astype(np.uint8)
+            s = np.full((rows, cols // 128), 0.02, np.float16)
+        q = np.ascontiguousarray(q)
+        s = np.ascontiguousarray(s) if s is not None else None
+        keep += [q, s]
+        ts.append(Tensor(name=name.encode(), kind=kind, rows=rows, cols=cols, data=q.ctypes.data, scale=s.ctypes.data if s is not None else None))
+    c = f.config
+    cfg = Config(hidden=c["hidden_size"], layers=c["num_hidden_layers"], heads=c["num_attention_heads"], kv_heads=c["num_key_value_heads"],
+                 head_dim=c["head_dim"], ffn=c["intermediate_size"], vocab=c["vocab_size"], tied=int(c["tie_embeddings"]),
+                 qkv_bias=int(c["qkv_bias"]), max_pos=c["max_position_embeddings"], rms_eps=c["rms_norm_eps"], rope_theta=c["rope_theta"])
+    h = C.c_void_p()
+    check(lib().qph_create(C.byref(cfg), (Tensor * len(ts))(*ts), len(ts), max_ctx, C.byref(h)))
+    f.close()
+    return qa.HipLlama(h.value)
+
+
+@pytest.mark.parametrize("n", [2, 40, 300])
+@pytest.mark.parametrize("kinds", [("q4", "q1", "q8"), ("q1", "q4", "q1"), ("q8", "q1", "q4"), ("q4", "q4", "q1"), ("q1", "q8", "q1")])
+def test_batched_prefill_mixed_qkv_kinds(kinds, n, synth, monkeypatch):
+    """q4 beside q1 among wq / wk / wv: their products read planes of different layouts from one buffer, so the activation
+    is quantised again between them - logits and cache rows of the batched prompt against this library's decode steps, which
+    read no planes, and against the reference order's kernels"""
+    path = synth("mini128")
+    shape = qa.CONFIGS["mini128"]
+    toks = np.random.default_rng(n).integers(0, shape.vocab, n).astype(np.int32)
+    gpu = with_kinds(path, dict(zip(("wq", "wk", "wv"), kinds)), n + 8)
+    print(f"q / k / v {kinds}: {n}-token prompt", flush=True)
+    out = []
+    for how in ("batched", "steps", "reference order"):
+        if how == "steps":
+            monkeypatch.setenv("QPH_PREFILL_STEPS", "1")
+        if how == "reference order":
+            monkeypatch.delenv("QPH_PREFILL_STEPS")
+            gpu.set_order(1)
+        gpu.reset()
+        out.append((gpu.prefill(toks, 1), split_snapshot(gpu.snapshot(), shape.layers, shape.kv_heads * shape.head_dim)))
+    gpu.close()
+    assert np.abs(out[0][0]).max() > 0.1
+    for lg, kv in out[1:]:
+        err, ok = close(out[0][0], lg)
+        assert ok, f"logits max|d| {err}"
+        for a, b in zip(out[0][1][1:], kv[1:]):
+            d = np.abs(a.astype(np.float32) - b.astype(np.float32))
+            assert d.max() <= 2e-3 * np.abs(b.astype(np.float32)).max(), float(d.max())
+
+
 @pytest.mark.parametrize("cfg,T,n", [("mini128", 900, 3), ("mini_r7h", 1500, 37), ("mini_r7", 800, 17), ("mini_q4m", 2000, 150),
                                      ("mini_odd", 750, 16)])
 @pytest.mark.parametrize("split", ["", "2", "31"])
