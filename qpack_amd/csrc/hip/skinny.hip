@@ -645,14 +645,19 @@ __global__ __launch_bounds__(kSkWaves * 64) void k_lowbit(GemmArgs a, int nrt, i
       lds_barrier();
       auto part = [&](int w, int tok, int row) { return *(const f4v *)(red + (w * RT16 + tok) * P + row); };
       auto sum = [&](int tok, int row) {
-        if constexpr (ORD) {
-          f4v v = (f4v){0.f, 0.f, 0.f, 0.f};
-          for (int w = 0; w < nb; w++) {
-            const f4v p = part(w, tok, row);
-            const float bs = bsl[w * NT + 16 * n0 + tok];
+        if constexpr (ORD) {   // no loop up to nb: its reads would wait for one another (pairs of 4864 x 896, 1024 tokens: 83 us, this 77)
+          f4v v = (f4v){0.f, 0.f, 0.f, 0.f}, p[kSkWaves];   // a wave without a block left zeros
+          float bs[kSkWaves];
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = __builtin_fmaf(bs, p[r], v[r]);
+          for (int w = 0; w < kSkWaves; w++) {
+            p[w] = part(w, tok, row);
+            const float b = bsl[min(w, nb - 1) * NT + 16 * n0 + tok];
+            bs[w] = w < nb ? b : 0.f;
           }
+#pragma unroll
+          for (int w = 0; w < kSkWaves; w++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = __builtin_fmaf(bs[w], p[w][r], v[r]);
           return v;
         } else {
           return ((part(0, tok, row) + part(1, tok, row)) + (part(2, tok, row) + part(3, tok, row))) +
