@@ -1123,7 +1123,7 @@ __global__ __launch_bounds__(kPfAttnWaves * 64) void k_pf_attn(PfAttnArgs a) {
 }
 // The splits' outputs of one (token, head) per wave, lane l holding dims HD / 64 l ..: M = max m, L = sum l 2^(m - M),
 // out = sum o 2^(m - M) / L in split order, stored or (a.oh) quantised as k_pf_attn does.  Bound by reading the partials
-// once (150 tokens x 28 heads x 12 splits: 26 MB).
+// once (150 tokens x 28 heads x 6 splits: 13 MB, 6 us).
 template <int HD>
 __global__ __launch_bounds__(256) void k_pf_attn_merge(PfAttnArgs a) {
   constexpr int D = HD / 64;
@@ -1171,13 +1171,17 @@ __global__ __launch_bounds__(256) void k_pf_attn_merge(PfAttnArgs a) {
 }
 
 // Splits of the cache per tile: few tokens behind a long context are a few dozen workgroups, each streaming the whole
-// cache at ~2.5 us per 64 positions (150 tokens, 28 heads in 4 groups at 12000: 36 workgroups, 430 us).  The split that is
-// expected to end first (here 6: 110 + 7 us): rounds of workgroups on the fullest XCD (the (group, share) pairs are dealt to the 8 XCDs, one
-// workgroup to a CU) times a share's blocks, then the merge (a launch and the partials); at least 4 blocks a share.
+// cache at ~2.5 us per 64 positions (150 tokens, 28 heads in 4 groups at 12000: 36 workgroups, 426 us).  The split that is
+// expected to end first (here 6: 94 + 6 us): rounds of workgroups on the fullest XCD (the (group, share) pairs are dealt to the 8 XCDs, one
+// workgroup to a CU) times a share's blocks, then the merge (a launch and the partials); at least 4 blocks a share.  What is
+// not expected to save 15 % is left unsplit, the expectation being that far off: 640 tokens behind 600 positions at 32 heads
+// in 8 groups, 53 us expected of three splits against 56, take 68 against 62.  Of 324 shapes (2 to 2048 tokens behind 0 to
+// 12000 positions, 14 / 2, 32 / 8 and 28 / 4 heads) no other split lost more than 2 %; the splits that are expected to save
+// less than 20 % saved 0 - 18 %, all others 7 - 92 %
 static int pf_attn_splits(int gx, int nkv, int blocks, int cus, int most) {
   const int per_xcd = std::max(1, cus / 8);
   int best = 1;
-  double tbest = (double)((gx * nkv + cus - 1) / cus) * (blocks + 2.5) * 2.5;
+  double tbest = 0.85 * ((gx * nkv + cus - 1) / cus) * (blocks + 2.5) * 2.5;
   for (int s = 2; s <= blocks / 4 && s <= most && s * gx * nkv <= 2 * cus; s++) {
     const int on_xcd = (nkv * s + 7) / 8 * gx;
     const double t = (double)((on_xcd + per_xcd - 1) / per_xcd) * ((blocks + s - 1) / s + 2.5) * 2.5 + 4 + 0.6 * s;
