@@ -17,7 +17,7 @@ struct DMat {
   const void *q;       // q8: int8 [rows, cols]; q4: u8 [rows, cols / 2]; q1: sign bits u8 [rows, cols / 8]; f32: float
   const void *s;       // q8: f32 [rows]; q4: fp16 [rows, cols / 32]; q1: fp16 [rows, cols / 128]
   int rows, cols, kind;
-  // layer matrices on the batched prompt path: q8 row sums per 128-column block [rows, cols / 128]; q4 / q1 the scales
+  // layer matrices on the batched prompt path: 128 x the q8 row sums per 128-column block (launch_rowsum_q8); q4 / q1 the scales
   // block-major (launch_scale_blocks)
   const int *rs;
   const uint16_t *st;

@@ -197,7 +197,7 @@ struct PfQuantArgs {
 };
 hipError_t launch_pf_quant(int pro, const PfQuantArgs &a, int B, hipStream_t st);
 // Y[t][r] = the row's dot product with token t's quantised activation (+ bias[r]), or Y[t][r] += that when resid.
-//   kind MK_Q8: w int8 [rows][cols], scale f32 [rows], wsum = row sums per 128-column block [rows][ldw] (launch_rowsum_q8)
+//   kind MK_Q8: w int8 [rows][cols], scale f32 [rows], wsum = 128 x its row sums per 128-column block (launch_rowsum_q8)
 //   kind MK_Q4 / MK_Q1: w as stored, the scales block-major in st, the activation's planes fp in the kind's order
 // one matrix of a multi-matrix product launch (GemmArgs::nseg > 1): its own weights, scales, bias and output
 struct GemmSeg {
@@ -240,11 +240,11 @@ struct GemmArgs {
 size_t gemm_lds_bytes();
 // row pitch of the block-major row sums: rows rounded up to 64 (16-byte loads of 4 rows stay inside a block's run)
 __host__ __device__ inline int ws_pitch(int rows) { return (rows + 63) & ~63; }
-// out[row][block] = sum of W[row] over each 128-column block
 // bytes [off, off + len) of a snapshot's body (per layer the first nb bytes of its K cache, then of its V cache; layers
 // `layer` bytes apart) -> out, which may be pinned host memory.  All sizes are multiples of 16
 hipError_t launch_cache_gather(const uint16_t *kc, const uint16_t *vc, size_t layer, size_t nb, size_t off, size_t len, void *out,
                                hipStream_t st);
+// out: 128 x the sum of W[row] over each 128-column block, [cols / 128][ws_pitch(rows)]
 hipError_t launch_rowsum_q8(const int8_t *w, int rows, int cols, int *out, hipStream_t st);
 // launch_gemm runs a q8 launch with th set on the few-token kernel, others on the tiled ones (which read xh / xl);
 // gemm_wants_tiles: whether th is the faster choice for this product (the pointers need not be set yet)
@@ -252,7 +252,7 @@ hipError_t launch_gemm(const GemmArgs &a, hipStream_t st);
 bool gemm_wants_tiles(const GemmArgs &a);
 // whether launch_gemm runs this q8 launch on the 32 x 32 kernel (the one that can quantise a SwiGLU pair's output)
 bool gemm_uses_32x32(const GemmArgs &a);
-// q4 / q1 products on the f16 matrix cores (skinny.hip): 16 rt rows (8 of each matrix of a pair) x 16 ntt tokens a tile
+// q4 products on the f16 matrix cores, q1 ones on the int8 cores (skinny.hip): 16 rt rows (8 of each matrix of a pair) x 16 ntt tokens a tile
 hipError_t launch_lowbit(const GemmArgs &a, int cus, hipStream_t st);
 // scales [rows][G] -> [block][row][4] (q4) or [block][row] (q1)
 hipError_t launch_scale_blocks(int kind, const uint16_t *sc, int rows, int cols, uint16_t *out, hipStream_t st);

@@ -9,7 +9,7 @@
 // A wave keeps the first 64 E keys it has seen (64 E >= M) sorted in registers, E per lane.  It sorts the next 64 E the
 // other way round (bitonic, lane exchanges by DPP and swizzles), keeps the smaller of each pair - the smallest 64 E of
 // both, a bitonic sequence - and sorts that in log2(64 E) stages; keys none of which precedes the list's last are
-// skipped.  A workgroup's 16 lists are merged pairwise in the same way through LDS, four barriers in all.  It is a chain of
+// skipped.  A workgroup's 16 lists are merged pairwise in the same way through LDS, two barriers for each of the four levels.  It is a chain of
 // lane exchanges, so its latency bounds it.  Measured (MI355X, 151936 values, us): M = 40 14 + 5, M = 100 15 + 9, M = 200 17 +
 // 18, M = 512 26 + 44 (before: a bitonic sort of 4096 keys per workgroup in LDS, 78 barriers and 28 - 32 us for each of two
 // rounds, three at M = 512).
